@@ -327,6 +327,10 @@ bool expert_gateup(const MoeArgs &a, int n_slots, hipStream_t st, hipEvent_t ev0
 void expert_down(const MoeArgs &a, int n_slots, hipStream_t st, bool mid_done = false);
 /* the down kernel alone on already quantized pair activations (a.mid) */
 void expert_down_q(const MoeArgs &a, int n_slots, hipStream_t st);
+/* the products of more tokens than k_gemm.hip's kernels take (k_mm.hip) */
+void mm_dense(const GemmArgs &a, hipStream_t st);
+void mm_gateup(const MoeArgs &a, int n_slots, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1);
+void mm_down(const MoeArgs &a, int n_slots, hipStream_t st);
 /* MLA: latent post step, absorbed queries, RoPE score term, output gather */
 void mla_post(const MlaArgs &a, hipStream_t st);
 void mla_qlat(const MlaArgs &a, hipStream_t st);

@@ -75,137 +75,6 @@ __device__ __forceinline__ void unpack_q4(v4i raw, v4i &a0, v4i &a1) {
     a1.x = raw.z & LO4; a1.y = raw.w & LO4; a1.z = (raw.z >> 4) & LO4; a1.w = (raw.w >> 4) & LO4;
 }
 
-/* Folds blocks [0, nb) of row tile rt of m against NT*16 tokens starting at token
- * index t0 (token t's activation row is row_of(t); tokens >= n read row_of(n - 1) and
- * their results are discarded). acc[tt][i] holds (row rt*16 + 4*(lane/16) + i,
- * token t0 + tt*16 + lane%16).
- *
- * A wave walks K one block pair at a time; the loads of pair gp + 1 (weights, scales,
- * the tokens' activation blocks and their scales) are issued before pair gp is folded,
- * so each pair's loads wait behind the previous pair's MFMAs and folds instead of
- * stalling the wave. */
-template <int NT>
-struct FoldStage {
-    v4i w0, w1;          /* Q8: the two blocks; Q4: w0 the packed pair */
-    uint2 s0, s1;        /* the blocks' f16 scales of this lane's 4 rows */
-    v4i b[2][NT];        /* activation blocks (16 bytes of each token's block) */
-    float dx[2][NT];
-    int sx[2][NT];       /* Q4: the activation block sums */
-};
-
-template <int NT>
-__device__ __forceinline__ void fold_load(FoldStage<NT> &f, const QMat &m, int rt, const Act &a, int gp,
-                                          const int (&arow)[NT], const uint16_t *dcol) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4, npair = m.nbp >> 1;
-    if (m.dtype == 4) {
-        f.w0 = load16(m.w + ((size_t)rt * npair + gp) * 1024 + lane * 16);
-    } else {
-        const uint8_t *base = m.w + ((size_t)rt * m.nbp + 2 * gp) * 1024 + lane * 16;
-        f.w0 = load16(base);
-        f.w1 = load16(base + 1024);
-    }
-    f.s0 = *(const uint2 *)(dcol + (size_t)(2 * gp) * m.rows_pad);
-    f.s1 = *(const uint2 *)(dcol + (size_t)(2 * gp + 1) * m.rows_pad);
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int g = 2 * gp + j < m.nb ? 2 * gp + j : m.nb - 1;   /* a pad block is never folded */
-#pragma unroll
-        for (int tt = 0; tt < NT; tt++) {
-            const size_t ab = (size_t)arow[tt] * a.nbp + g;
-            f.b[j][tt] = load16((const uint8_t *)(a.q + ab * 64 + kg * 16));
-            f.dx[j][tt] = a.d[ab];
-            if (m.dtype == 4) f.sx[j][tt] = a.s[ab];
-        }
-    }
-}
-
-template <int NT, typename RowOf>
-__device__ __forceinline__ void fold_tile(const QMat &m, int rt, const Act &a, int t0, int n, RowOf row_of,
-                                          float (&acc)[NT][4]) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4, lr = lane & 15;
-    int arow[NT];
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++) {
-        int t = t0 + tt * 16 + lr;
-        t = t < n ? t : n - 1;
-        arow[tt] = row_of(t);
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[tt][i] = 0.0f;
-    }
-    const v4i zero = {0, 0, 0, 0};
-    const int npair = m.nbp >> 1;
-    const uint16_t *dcol = m.d + rt * 16 + 4 * kg;
-    FoldStage<NT> cur, nxt;
-    fold_load<NT>(cur, m, rt, a, 0, arow, dcol);
-    for (int gp = 0; gp < npair; gp++) {
-        if (gp + 1 < npair) fold_load<NT>(nxt, m, rt, a, gp + 1, arow, dcol);
-        v4i w0 = cur.w0, w1 = cur.w1;
-        if (m.dtype == 4) unpack_q4(cur.w0, w0, w1);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int g = 2 * gp + j;
-            if (g >= m.nb) break;
-            const uint2 sw = j ? cur.s1 : cur.s0;
-            float dw[4];
-            dw[0] = h2f((uint16_t)(sw.x & 0xffff));
-            dw[1] = h2f((uint16_t)(sw.x >> 16));
-            dw[2] = h2f((uint16_t)(sw.y & 0xffff));
-            dw[3] = h2f((uint16_t)(sw.y >> 16));
-            const v4i wa = j ? w1 : w0;
-#pragma unroll
-            for (int tt = 0; tt < NT; tt++) {
-                v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa, cur.b[j][tt], zero, 0, 0, 0);
-                const float dx = cur.dx[j][tt];
-                if (m.dtype == 4) {
-                    const int off = 8 * cur.sx[j][tt];   /* sum(nib * q) - 8 sum(q) = sum((nib - 8) q) */
-                    c.x -= off; c.y -= off; c.z -= off; c.w -= off;
-                }
-                acc[tt][0] = fadd(acc[tt][0], fmul((float)c.x, fmul(dw[0], dx)));
-                acc[tt][1] = fadd(acc[tt][1], fmul((float)c.y, fmul(dw[1], dx)));
-                acc[tt][2] = fadd(acc[tt][2], fmul((float)c.z, fmul(dw[2], dx)));
-                acc[tt][3] = fadd(acc[tt][3], fmul((float)c.w, fmul(dw[3], dx)));
-            }
-        }
-        cur = nxt;
-    }
-}
-
-/* ------------------------------------------------------------ dense segmented GEMM */
-
-/* One wave per (16-row tile, group of NT 16-token tiles). Workgroup b covers row tiles
- * of workgroup-row b % wgr and token group b / wgr; wgr is a multiple of 8, so every
- * token group of a row tile runs on the same XCD (IDs are dealt round-robin to the 8
- * XCDs) and re-reads its weights from that XCD's L2. */
-template <int NT>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs args, int wgr) {
-    const int rw = (int)blockIdx.x % wgr, tg = (int)blockIdx.x / wgr;
-    int s = 0;
-    while (s + 1 < args.nseg && rw >= args.seg[s + 1].wg0) s++;
-    const GemmSeg &sg = args.seg[s];
-    if (rw >= sg.wg0 + (sg.m.rows_pad / 16 + 3) / 4) return;   /* padding workgroup */
-    const int rt = (rw - sg.wg0) * 4 + (int)(threadIdx.x >> 6);
-    if (rt * 16 >= sg.m.rows_pad) return;
-    const int t0 = args.t0 + tg * NT * 16;
-    if (t0 >= args.T) return;
-    float acc[NT][4];
-    fold_tile<NT>(sg.m, rt, args.a, t0, args.T, [](int t) { return t; }, acc);
-    const int lane = threadIdx.x & 63, kg = lane >> 4, lr = lane & 15;
-#pragma unroll
-    for (int tt = 0; tt < NT; tt++) {
-        const int t = t0 + tt * 16 + lr;
-        if (t >= args.T) continue;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = rt * 16 + 4 * kg + i;
-            if (row < sg.m.rows) {
-                float y = canon(acc[tt][i]);
-                if (sg.scale_on) y = canon(fmul(sg.scale, y));
-                sg.Y[(size_t)t * sg.ldy + row] = y;
-            }
-        }
-    }
-}
-
 /* ------------------------------------------------------------ split-K products (few tokens) */
 
 /* With few tokens a product is bound by how many weight bytes are in flight, not by the
@@ -342,109 +211,6 @@ __device__ __forceinline__ void wave_pairs(int npair, int W, int w, int &p0, int
     p1 = p0 + ppw < npair ? p0 + ppw : npair;
 }
 
-/* Resident split-K: a wave's weights and scales of NM matrices for its block pairs
- * [p0, p1) (at most SK_MAXP) stay in registers while token tiles pass through them;
- * skm_load_x loads one tile's activation blocks (row arow of a for this lane's token),
- * skm_terms writes the tile's terms as tile_terms_chunk does. */
-template <int DT, int NM>
-struct SkmRegs {
-    v4i raw[NM][SK_MAXP][DT == 4 ? 1 : 2];
-    uint2 sc[NM][SK_MAXP][2];
-    v4i xq[SK_MAXP][2];
-    float dx[SK_MAXP][2];
-    int sx[SK_MAXP][2];
-};
-
-template <int DT, int NM>
-__device__ __forceinline__ void skm_load_w(SkmRegs<DT, NM> &r, const QMat *ms, int rt, int p0, int p1) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4;
-    const int npair = ms[0].nbp >> 1;
-#pragma unroll
-    for (int k = 0; k < SK_MAXP; k++) {
-        const int gp = p0 + k < p1 ? p0 + k : p1 - 1;
-#pragma unroll
-        for (int mi = 0; mi < NM; mi++) {
-            const QMat &m = ms[mi];
-            if (DT == 4) {
-                r.raw[mi][k][0] = load16(m.w + ((size_t)rt * npair + gp) * 1024 + lane * 16);
-            } else {
-                const uint8_t *base = m.w + ((size_t)rt * m.nbp + 2 * gp) * 1024 + lane * 16;
-                r.raw[mi][k][0] = load16(base);
-                r.raw[mi][k][DT == 4 ? 0 : 1] = load16(base + 1024);
-            }
-            const uint16_t *dcol = m.d + rt * 16 + 4 * kg;
-            r.sc[mi][k][0] = *(const uint2 *)(dcol + (size_t)(2 * gp) * m.rows_pad);
-            r.sc[mi][k][1] = *(const uint2 *)(dcol + (size_t)(2 * gp + 1) * m.rows_pad);
-        }
-    }
-}
-
-template <int DT, int NM>
-__device__ __forceinline__ void skm_load_x(SkmRegs<DT, NM> &r, const Act &a, int arow, int p0, int p1) {
-    const int kg = (threadIdx.x & 63) >> 4;
-#pragma unroll
-    for (int k = 0; k < SK_MAXP; k++) {
-        const int gp = p0 + k < p1 ? p0 + k : p1 - 1;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const size_t ab = (size_t)arow * a.nbp + 2 * gp + j;
-            r.xq[k][j] = load16((const uint8_t *)(a.q + ab * 64 + kg * 16));
-            r.dx[k][j] = a.d[ab];
-            r.sx[k][j] = DT == 4 ? a.s[ab] : 0;
-        }
-    }
-}
-
-template <int DT, int NM>
-__device__ __forceinline__ void skm_terms(const SkmRegs<DT, NM> &r, int nb, int ntok, int p0, int p1, float *P,
-                                          int pstride) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4, lr = lane & 15;
-    const v4i zero = {0, 0, 0, 0};
-    float *dmy = P + (size_t)NM * nb * ntok * 16 + lane * 4;   /* after the NM matrices' terms */
-    /* one matrix at a time: its MFMAs first (each into its own registers), then its f32
-     * terms, so no term waits on the MFMA just issued */
-#pragma unroll
-    for (int mi = 0; mi < NM; mi++) {
-        v4i cc[SK_MAXP][2];
-#pragma unroll
-        for (int k = 0; k < SK_MAXP; k++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                v4i wa;
-                if (DT == 4) {
-                    v4i w0, w1;
-                    unpack_q4(r.raw[mi][k][0], w0, w1);
-                    wa = j ? w1 : w0;
-                } else {
-                    wa = r.raw[mi][k][DT == 4 ? 0 : j];
-                }
-                cc[k][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa, r.xq[k][j], zero, 0, 0, 0);
-            }
-#pragma unroll
-        for (int k = 0; k < SK_MAXP; k++) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int g = 2 * (p0 + k) + j;
-                if (p0 + k >= p1 || g >= nb) continue;   /* uniform */
-                v4i c = cc[k][j];
-                if (DT == 4) {
-                    const int off = 8 * r.sx[k][j];   /* sum(nib * q) - 8 sum(q) = sum((nib - 8) q) */
-                    c.x -= off; c.y -= off; c.z -= off; c.w -= off;
-                }
-                const uint2 sw = r.sc[mi][k][j];
-                const float d = r.dx[k][j];
-                float4 v;
-                v.x = fmul((float)c.x, fmul(h2f((uint16_t)(sw.x & 0xffff)), d));
-                v.y = fmul((float)c.y, fmul(h2f((uint16_t)(sw.x >> 16)), d));
-                v.z = fmul((float)c.z, fmul(h2f((uint16_t)(sw.y & 0xffff)), d));
-                v.w = fmul((float)c.w, fmul(h2f((uint16_t)(sw.y >> 16)), d));
-                float *dst = lr < ntok ? P + (size_t)mi * pstride + ((size_t)g * ntok + lr) * 16 + 4 * kg : dmy;
-                *(float4 *)dst = v;
-            }
-        }
-    }
-}
-
 /* dense product of few tokens: one workgroup per 16-row tile of a segment. */
 template <int DT>
 __global__ __launch_bounds__(512) void k_gemm_sk(GemmArgs args, int ntok) {
@@ -476,267 +242,6 @@ __global__ __launch_bounds__(512) void k_gemm_sk(GemmArgs args, int ntok) {
             }
         }
         __syncthreads();
-    }
-}
-
-/* Dense product of more tokens than one tile (a tree's, a prefill chunk's) with each
- * weight byte read once: one workgroup per 16-row tile of a segment, as k_gemm_sk; each
- * wave keeps the weights and scales of its block pairs (at most SK_MAXP) in registers
- * and runs every token tile through them: the MFMAs, the terms into LDS, the next
- * tile's activation loads (in flight during the barrier and the fold), one thread per
- * (row, token) folding the terms in block order. The same terms and fold as k_gemm_sk,
- * so the same bits as every other product kernel. */
-template <int DT>
-__global__ __launch_bounds__(512) void k_gemm_skm(GemmArgs args, int ntok, int nwg, int nsplit) {
-    extern __shared__ float P[];
-    /* workgroup b takes row tile b % nwg and token tiles b / nwg, b / nwg + nsplit, ... */
-    const int bid = (int)blockIdx.x % nwg, split = (int)blockIdx.x / nwg;
-    int s = 0;
-    while (s + 1 < args.nseg && bid >= args.seg[s + 1].wg0) s++;
-    const GemmSeg &sg = args.seg[s];
-    const QMat &m = sg.m;
-    const int rt = bid - sg.wg0;
-    const int tfirst = args.t0 + split * ntok, tstep = nsplit * ntok;
-    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x, lr = tid & 15;
-    int p0, p1;
-    wave_pairs(m.nbp >> 1, W, wave, p0, p1);
-    const bool has = p0 < p1;   /* uniform per wave */
-    auto arow = [&](int t0) { const int t = t0 + lr; return t < args.T ? t : args.T - 1; };
-    SkmRegs<DT, 1> r;
-    if (has) {
-        skm_load_w<DT, 1>(r, &m, rt, p0, p1);
-        if (tfirst < args.T) skm_load_x<DT, 1>(r, args.a, arow(tfirst), p0, p1);
-    }
-    for (int t0 = tfirst; t0 < args.T; t0 += tstep) {
-        if (has) {
-            skm_terms<DT, 1>(r, m.nb, ntok, p0, p1, P, 0);
-            if (t0 + tstep < args.T) skm_load_x<DT, 1>(r, args.a, arow(t0 + tstep), p0, p1);
-        }
-        __syncthreads();
-        for (int f = tid; f < ntok * 16; f += blockDim.x) {
-            const int c = f >> 4, row = rt * 16 + (f & 15), t = t0 + c;
-            const float acc = fold_terms(P, m.nb, ntok, f);
-            if (t < args.T && row < m.rows) {
-                float y = canon(acc);
-                if (sg.scale_on) y = canon(fmul(sg.scale, y));
-                sg.Y[(size_t)t * sg.ldy + row] = y;
-            }
-        }
-        __syncthreads();
-    }
-}
-
-/* gate/up with resident weights: a slot's gate and up weights are read once and every
- * token tile of the slot runs through them (as k_gemm_skm); for waves of at most SK_MAXP
- * block pairs and 4 waves a workgroup, held to 256 VGPRs (two waves per SIMD: with
- * 272 the kernel ran one and was slower than reloading the weights per tile) */
-template <int DT>
-__global__ __launch_bounds__(256, 2) void k_expert_gateup_skm(MoeArgs a, int ntok) {
-    extern __shared__ float P[];
-    const int ntile = a.F / 16;
-    const int u = (int)blockIdx.x / ntile, rt = (int)blockIdx.x % ntile;
-    const SlotDesc &sd = a.desc[u];
-    const int n = sd.n, p0 = sd.p0;
-    if (n == 0) return;
-    const ExpertW ew = sd.w;
-    if (ew.gate.dtype != DT) return;   /* the launcher runs one instantiation per dtype */
-    const QMat ms[2] = {ew.gate, ew.up};
-    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x, lr = tid & 15;
-    int q0, q1;
-    wave_pairs(ew.gate.nbp >> 1, W, wave, q0, q1);
-    const bool has = q0 < q1;
-    const int nb = ew.gate.nb, pstride = nb * ntok * 16;
-    const int *ptok = a.pair_tok + p0;
-    auto arow = [&](int t0) { const int t = t0 + lr; return ptok[t < n ? t : n - 1]; };
-    SkmRegs<DT, 2> r;
-    if (has) {
-        skm_load_w<DT, 2>(r, ms, rt, q0, q1);
-        skm_load_x<DT, 2>(r, a.x, arow(0), q0, q1);
-    }
-    for (int t0 = 0; t0 < n; t0 += ntok) {
-        if (has) {
-            skm_terms<DT, 2>(r, nb, ntok, q0, q1, P, pstride);
-            if (t0 + ntok < n) skm_load_x<DT, 2>(r, a.x, arow(t0 + ntok), q0, q1);
-        }
-        __syncthreads();
-        for (int f = tid; f < ntok * 16; f += blockDim.x) {
-            const int c = f >> 4, row = rt * 16 + (f & 15);
-            const float gv = canon(fold_terms(P, nb, ntok, f));
-            const float uv = canon(fold_terms(P + pstride, nb, ntok, f));
-            if (t0 + c < n) {
-                const float sg = fdiv(gv, fadd(1.0f, exp_glibc_f(-gv)));
-                a.midf[(size_t)(p0 + t0 + c) * a.F + row] = fmul(sg, uv);
-            }
-        }
-        __syncthreads();
-    }
-}
-
-/* gate/up of one 16-row F tile of one active expert for its n tokens, then
- * mid = silu(g) * u (NUMERICS §4, quant.c:644-649) as f32 [pair][F]. */
-template <int DT>
-__global__ __launch_bounds__(512) void k_expert_gateup_sk(MoeArgs a, int ntok) {
-    extern __shared__ float P[];
-    const int ntile = a.F / 16;
-    const int u = (int)blockIdx.x / ntile, rt = (int)blockIdx.x % ntile;
-    const SlotDesc &sd = a.desc[u];
-    const int n = sd.n, p0 = sd.p0;
-    if (n == 0) return;
-    const ExpertW ew = sd.w;
-    if (ew.gate.dtype != DT) return;   /* the launcher runs one instantiation per dtype */
-    const QMat ms[2] = {ew.gate, ew.up};
-    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x;
-    int q0, q1;
-    wave_pairs(ew.gate.nbp >> 1, W, wave, q0, q1);
-    const int pstride = ew.gate.nb * ntok * 16;
-    const int *ptok = a.pair_tok + p0;
-    for (int t0 = 0; t0 < n; t0 += ntok) {
-        tile_terms<DT, 2>(ms, rt, a.x, t0, n, ntok, [ptok](int t) { return ptok[t]; }, q0, q1, P, pstride);
-        __syncthreads();
-        for (int f = tid; f < ntok * 16; f += blockDim.x) {
-            const int c = f >> 4, row = rt * 16 + (f & 15);
-            const float gv = canon(fold_terms(P, ew.gate.nb, ntok, f));
-            const float uv = canon(fold_terms(P + pstride, ew.gate.nb, ntok, f));
-            if (t0 + c < n) {
-                const float sg = fdiv(gv, fadd(1.0f, exp_glibc_f(-gv)));
-                a.midf[(size_t)(p0 + t0 + c) * a.F + row] = fmul(sg, uv);
-            }
-        }
-        __syncthreads();
-    }
-}
-
-/* Persistent gate/up for few tokens (every expert's tokens fit one token tile and a
- * wave's pair range fits SK_MAXP): workgroups loop over the items (active slot, 16-row
- * F tile); as soon as an item's MFMAs have consumed its operand registers, the next
- * item's loads are issued into them, and the barrier, the ordered fold and the SwiGLU
- * epilogue of the current item run while those bytes are in flight. */
-template <int DT>
-__device__ __forceinline__ void gu_issue(const SlotDesc &sd, int rt, const Act &a, const int *pair_tok, int q0,
-                                         int q1, v4i (&rw)[2][SK_MAXP][DT == 4 ? 1 : 2], uint2 (&sc)[2][SK_MAXP][2],
-                                         v4i (&xq)[SK_MAXP][2], float (&dx)[SK_MAXP][2], int (&sx)[SK_MAXP][2]) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4, lr = lane & 15;
-    const int n = sd.n;
-    const int arow = pair_tok[sd.p0 + (lr < n ? lr : n - 1)];
-    const int npair = sd.w.gate.nbp >> 1;
-#pragma unroll
-    for (int k = 0; k < SK_MAXP; k++) {
-        const int gp = q0 + k < q1 ? q0 + k : q1 - 1;
-#pragma unroll
-        for (int mi = 0; mi < 2; mi++) {
-            const QMat &m = mi ? sd.w.up : sd.w.gate;
-            if (DT == 4) {
-                rw[mi][k][0] = load16(m.w + ((size_t)rt * npair + gp) * 1024 + lane * 16);
-            } else {
-                const uint8_t *base = m.w + ((size_t)rt * m.nbp + 2 * gp) * 1024 + lane * 16;
-                rw[mi][k][0] = load16(base);
-                rw[mi][k][DT == 4 ? 0 : 1] = load16(base + 1024);
-            }
-            const uint16_t *dcol = m.d + rt * 16 + 4 * kg;
-            sc[mi][k][0] = *(const uint2 *)(dcol + (size_t)(2 * gp) * m.rows_pad);
-            sc[mi][k][1] = *(const uint2 *)(dcol + (size_t)(2 * gp + 1) * m.rows_pad);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const size_t ab = (size_t)arow * a.nbp + 2 * gp + j;
-            xq[k][j] = load16((const uint8_t *)(a.q + ab * 64 + kg * 16));
-            dx[k][j] = a.d[ab];
-            sx[k][j] = DT == 4 ? a.s[ab] : 0;
-        }
-    }
-}
-
-template <int DT>
-__device__ __forceinline__ void gu_terms(int nb, int ntok, int q0, int q1, const v4i (&rw)[2][SK_MAXP][DT == 4 ? 1 : 2],
-                                         const uint2 (&sc)[2][SK_MAXP][2], const v4i (&xq)[SK_MAXP][2],
-                                         const float (&dx)[SK_MAXP][2], const int (&sx)[SK_MAXP][2], float *P,
-                                         int pstride) {
-    const int lane = threadIdx.x & 63, kg = lane >> 4, lr = lane & 15;
-    const v4i zero = {0, 0, 0, 0};
-    v4i cc[2][SK_MAXP][2];
-#pragma unroll
-    for (int k = 0; k < SK_MAXP; k++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int mi = 0; mi < 2; mi++) {
-                v4i wa;
-                if (DT == 4) {
-                    v4i w0, w1;
-                    unpack_q4(rw[mi][k][0], w0, w1);
-                    wa = j ? w1 : w0;
-                } else {
-                    wa = rw[mi][k][DT == 4 ? 0 : j];
-                }
-                cc[mi][k][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa, xq[k][j], zero, 0, 0, 0);
-            }
-    float *dmy = P + (size_t)2 * nb * ntok * 16 + lane * 4;   /* after both matrices' terms */
-#pragma unroll
-    for (int k = 0; k < SK_MAXP; k++) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int g = 2 * (q0 + k) + j;
-            if (q0 + k >= q1 || g >= nb) continue;   /* uniform */
-#pragma unroll
-            for (int mi = 0; mi < 2; mi++) {
-                v4i c = cc[mi][k][j];
-                if (DT == 4) {
-                    const int off = 8 * sx[k][j];
-                    c.x -= off; c.y -= off; c.z -= off; c.w -= off;
-                }
-                const uint2 sw = sc[mi][k][j];
-                const float d = dx[k][j];
-                float4 v;
-                v.x = fmul((float)c.x, fmul(h2f((uint16_t)(sw.x & 0xffff)), d));
-                v.y = fmul((float)c.y, fmul(h2f((uint16_t)(sw.x >> 16)), d));
-                v.z = fmul((float)c.z, fmul(h2f((uint16_t)(sw.y & 0xffff)), d));
-                v.w = fmul((float)c.w, fmul(h2f((uint16_t)(sw.y >> 16)), d));
-                float *dst = lr < ntok ? P + (size_t)mi * pstride + ((size_t)g * ntok + lr) * 16 + 4 * kg : dmy;
-                *(float4 *)dst = v;
-            }
-        }
-    }
-}
-
-template <int DT>
-__global__ __launch_bounds__(256) void k_expert_gateup_pp(MoeArgs a, int ntok) {
-    extern __shared__ float P[];
-    const int ntile = a.F / 16;
-    const int n_items = *a.n_active * ntile;
-    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x;
-    int item = blockIdx.x;
-    if (item >= n_items) return;   /* uniform */
-    v4i rw[2][SK_MAXP][DT == 4 ? 1 : 2];
-    uint2 sc[2][SK_MAXP][2];
-    v4i xq[SK_MAXP][2];
-    float dx[SK_MAXP][2];
-    int sx[SK_MAXP][2];
-    const SlotDesc *sd = &a.desc[item / ntile];
-    int q0, q1;
-    wave_pairs(sd->w.gate.nbp >> 1, W, wave, q0, q1);
-    gu_issue<DT>(*sd, item % ntile, a.x, a.pair_tok, q0, q1, rw, sc, xq, dx, sx);
-    while (item < n_items) {
-        const int rt = item % ntile, p0 = sd->p0, n = sd->n, nb = sd->w.gate.nb;
-        const int pstride = nb * ntok * 16;
-        if (sd->w.gate.dtype == DT) gu_terms<DT>(nb, ntok, q0, q1, rw, sc, xq, dx, sx, P, pstride);
-        const int next = item + (int)gridDim.x;
-        const SlotDesc *nsd = &a.desc[(next < n_items ? next : item) / ntile];
-        if (next < n_items) gu_issue<DT>(*nsd, next % ntile, a.x, a.pair_tok, q0, q1, rw, sc, xq, dx, sx);
-        __syncthreads();
-        if (sd->w.gate.dtype == DT) {
-            for (int f = tid; f < ntok * 16; f += blockDim.x) {
-                const int c = f >> 4, row = rt * 16 + (f & 15);
-                const float gv = canon(fold_terms(P, nb, ntok, f));
-                const float uv = canon(fold_terms(P + pstride, nb, ntok, f));
-                if (c < n) {
-                    const float sg = fdiv(gv, fadd(1.0f, exp_glibc_f(-gv)));
-                    a.midf[(size_t)(p0 + c) * a.F + row] = fmul(sg, uv);
-                }
-            }
-        }
-        __syncthreads();
-        item = next;
-        sd = nsd;
     }
 }
 
@@ -1064,43 +569,6 @@ int launch_tk(const MoeArgs &a, int mode, int n_slots, hipStream_t st, hipEvent_
     return qf ? 2 : 1;
 }
 
-/* down projection of one 16-row D tile of one active expert for its n tokens. */
-template <int DT>
-__global__ __launch_bounds__(512) void k_expert_down_sk(MoeArgs a, int ntok) {
-    extern __shared__ float P[];
-    const int ntile = (a.D + 15) / 16;
-    const int u = (int)blockIdx.x / ntile, rt = (int)blockIdx.x % ntile;
-    int n, p0;
-    QMat m;
-    if (a.head_slots) {
-        n = a.T;
-        p0 = u * a.T;
-        m = a.table[u].down;
-    } else {
-        const SlotDesc &sd = a.desc[u];
-        n = sd.n;
-        p0 = sd.p0;
-        m = sd.w.down;
-    }
-    if (n == 0) return;
-    if (m.dtype != DT) return;
-    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x;
-    int q0, q1;
-    wave_pairs(m.nbp >> 1, W, wave, q0, q1);
-    for (int t0 = 0; t0 < n; t0 += ntok) {
-        tile_terms<DT, 1>(&m, rt, a.mid, t0, n, ntok, [p0](int t) { return p0 + t; }, q0, q1, P, 0);
-        __syncthreads();
-        for (int f = tid; f < ntok * 16; f += blockDim.x) {
-            const int c = f >> 4, row = rt * 16 + (f & 15);
-            const float acc = fold_terms(P, m.nb, ntok, f);
-            if (t0 + c < n && row < m.rows) a.Y[(size_t)(p0 + t0 + c) * a.D + row] = canon(acc);
-        }
-        __syncthreads();
-    }
-}
-
-/* ------------------------------------------------------------ grouped expert GEMMs */
-
 /* ------------------------------------------------------------ float matrices (dot16) */
 
 /* y = dot16(w_r, x_t) (NUMERICS §1/§3; quant.c:352-376): 16 lanes per (row, token),
@@ -1221,18 +689,6 @@ void quant_rows(const float *x, int64_t ldx, int T, int nb, const Act &a, hipStr
     k_quant_rows<<<(int)((waves + 3) / 4), 256, 0, st>>>(x, ldx, T, nb, a);
 }
 
-/* compute units of the current device (cached per device) */
-static int cu_count() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cached[dev]) {
-        int n = 0;
-        cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-    }
-    return cached[dev];
-}
-
 /* waves per split-K workgroup for npair block pairs */
 static int sk_waves(int npair) {
     const int w = (npair + SK_MAXP - 1) / SK_MAXP;
@@ -1247,19 +703,9 @@ static int sk_ntok(int T, int NM, int nb) {
     return n < 1 ? 1 : n;
 }
 
-/* k_gemm_skm applies: every segment's block pairs fit its waves' registers (at most 8
- * waves of SK_MAXP pairs) and its terms the LDS */
-static bool skm_ok(const GemmArgs &in) {
-    for (int s = 0; s < in.nseg; s++) {
-        const QMat &m = in.seg[s].m;
-        if ((m.nbp >> 1) > 8 * SK_MAXP || (size_t)m.nb * 64 > (size_t)SK_LDS) return false;
-    }
-    return true;
-}
-
-/* dense product through the split-K kernels (k_gemm_sk, or k_gemm_skm when resident):
- * one launch per run of consecutive segments of one dtype */
-static void gemm_sk(const GemmArgs &in, hipStream_t st, bool resident = false) {
+/* dense product through the split-K kernel: one launch per run of consecutive segments of
+ * one dtype */
+static void gemm_sk(const GemmArgs &in, hipStream_t st) {
     for (int s0 = 0; s0 < in.nseg;) {
         int s1 = s0 + 1;
         while (s1 < in.nseg && in.seg[s1].m.dtype == in.seg[s0].m.dtype && in.seg[s1].m.nb == in.seg[s0].m.nb) s1++;
@@ -1275,14 +721,7 @@ static void gemm_sk(const GemmArgs &in, hipStream_t st, bool resident = false) {
         const int ntok = sk_ntok(in.T, 1, m.nb);
         const int threads = 64 * sk_waves(m.nbp / 2);
         const size_t lds = (size_t)m.nb * ntok * 64 + SK_DUMMY;
-        if (wg && resident) {
-            /* token tiles split over workgroups until the row tiles fill the CUs */
-            const int ntile = (in.T + ntok - 1) / ntok;
-            int nsplit = 1;
-            while (nsplit < ntile && wg * (nsplit + 1) <= cu_count()) nsplit++;
-            if (m.dtype == 4) k_gemm_skm<4><<<wg * nsplit, threads, lds, st>>>(g, ntok, wg, nsplit);
-            else k_gemm_skm<3><<<wg * nsplit, threads, lds, st>>>(g, ntok, wg, nsplit);
-        } else if (wg) {
+        if (wg) {
             if (m.dtype == 4) k_gemm_sk<4><<<wg, threads, lds, st>>>(g, ntok);
             else k_gemm_sk<3><<<wg, threads, lds, st>>>(g, ntok);
         }
@@ -1291,71 +730,22 @@ static void gemm_sk(const GemmArgs &in, hipStream_t st, bool resident = false) {
 }
 
 void gemm(const GemmArgs &in, hipStream_t st) {
-    if (in.T <= 16 && in.t0 == 0) {
-        bool ok = true;
-        for (int s = 0; s < in.nseg; s++) ok = ok && (size_t)in.seg[s].m.nb * 64 <= (size_t)SK_LDS;
-        if (ok) { gemm_sk(in, st); return; }
-    }
-    if (in.t0 == 0 && skm_ok(in)) { gemm_sk(in, st, true); return; }
-    GemmArgs g = in;
-    int wg = 0, tiles = 0;
-    for (int s = 0; s < g.nseg; s++) {
-        g.seg[s].wg0 = wg;
-        wg += (g.seg[s].m.rows_pad / 16 + 3) / 4;
-        tiles += g.seg[s].m.rows_pad / 16;
-    }
-    if (!wg || in.T <= 0) return;
-    const int wgr = (wg + 7) & ~7;
-    /* tokens tiles per wave: as many as keep about 8 waves per CU busy (each wave walks
-     * all of K for its tiles, so more tiles per wave means fewer, longer waves) */
-    const int ntile = (in.T + 15) / 16, want = 8 * cu_count();
-    int nt = 8;
-    while (nt > 1 && (long long)tiles * ((ntile + nt - 1) / nt) < want) nt >>= 1;
-    if (nt > ntile) nt = ntile <= 1 ? 1 : ntile <= 2 ? 2 : ntile <= 4 ? 4 : 8;
-    g.t0 = 0;
-    const int grid = wgr * ((ntile + nt - 1) / nt);
-    if (nt == 1) k_gemm<1><<<grid, 256, 0, st>>>(g, wgr);
-    else if (nt == 2) k_gemm<2><<<grid, 256, 0, st>>>(g, wgr);
-    else if (nt == 4) k_gemm<4><<<grid, 256, 0, st>>>(g, wgr);
-    else k_gemm<8><<<grid, 256, 0, st>>>(g, wgr);
+    bool few = in.T <= 16;   /* k_gemm_sk's terms of at least one token fit its LDS */
+    for (int s = 0; s < in.nseg; s++) few = few && (size_t)in.seg[s].m.nb * 64 <= (size_t)(SK_LDS - SK_DUMMY);
+    if (few) gemm_sk(in, st);
+    else mm_dense(in, st);
 }
 
-/* gate/up (split-K, one launch per expert dtype present); true when the launch also
- * quantized the SwiGLU rows into a.mid */
+/* gate/up; true when the launch also quantized the SwiGLU rows into a.mid. ev0 / ev1
+ * (optional) are recorded by the dispatch itself: ev0 at the start of the first launch, ev1
+ * at the end of the last. */
 bool expert_gateup(const MoeArgs &a, int n_slots, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     if (n_slots <= 0) return false;
-    const int nb = (a.D + 63) / 64, nbp = (nb + 1) & ~1;
-    const int ntok = sk_ntok(a.T, 2, nb);
-    const int threads = 64 * sk_waves(nbp / 2);
-    const size_t lds = (size_t)2 * nb * ntok * 64 + SK_DUMMY;
-    const int grid = n_slots * (a.F / 16);
-    /* ev0/ev1 (optional) are recorded by the dispatch itself: ev0 at the start of the
-     * first launch, ev1 at the end of the last */
-    const bool q4 = a.dtype_mask & (1 << 4), q8 = a.dtype_mask & (1 << 3);
-    /* at most 16 tokens per expert, one dtype: the split-K kernel (one term per lane) */
+    /* at most 16 tokens per expert, one dtype, token blocks within its LDS: the split-K
+     * kernel (one term per lane); else the chunked one */
     if (const int r = launch_tk(a, TK_GATEUP, n_slots, st, ev0, ev1)) return r == 2;
-    /* few tokens, one dtype, one pair chunk per wave: the persistent kernel (two
-     * workgroups per CU on every CU) */
-    const int npair = nbp / 2, W = threads / 64;
-    if (a.T <= ntok && (q4 != q8) && (npair + W - 1) / W <= SK_MAXP && threads <= 256) {
-        const int ncu = cu_count();
-        const int pgrid = grid < 2 * ncu ? grid : 2 * ncu;
-        if (q4) hipExtLaunchKernelGGL(k_expert_gateup_pp<4>, dim3(pgrid), dim3(threads), (uint32_t)lds, st, ev0, ev1, 0u, a, ntok);
-        else hipExtLaunchKernelGGL(k_expert_gateup_pp<3>, dim3(pgrid), dim3(threads), (uint32_t)lds, st, ev0, ev1, 0u, a, ntok);
-        return false;
-    }
-    if ((npair + W - 1) / W <= SK_MAXP && threads <= 256) {   /* the wave's pairs fit its registers */
-        if (q4) hipExtLaunchKernelGGL(k_expert_gateup_skm<4>, dim3(grid), dim3(threads), (uint32_t)lds, st, ev0,
-                                      q8 ? nullptr : ev1, 0u, a, ntok);
-        if (q8) hipExtLaunchKernelGGL(k_expert_gateup_skm<3>, dim3(grid), dim3(threads), (uint32_t)lds, st,
-                                      q4 ? nullptr : ev0, ev1, 0u, a, ntok);
-        return false;
-    }
-    if (q4) hipExtLaunchKernelGGL(k_expert_gateup_sk<4>, dim3(grid), dim3(threads), (uint32_t)lds, st, ev0,
-                                  q8 ? nullptr : ev1, 0u, a, ntok);
-    if (q8) hipExtLaunchKernelGGL(k_expert_gateup_sk<3>, dim3(grid), dim3(threads), (uint32_t)lds, st,
-                                  q4 ? nullptr : ev0, ev1, 0u, a, ntok);
-    return false;
+    mm_gateup(a, n_slots, st, ev0, ev1);
+    return true;
 }
 
 /* NUMERICS §2 of the SwiGLU rows of all T * top_k pairs (unless the gate/up launch did
@@ -1369,13 +759,7 @@ void expert_down(const MoeArgs &a, int n_slots, hipStream_t st, bool mid_done) {
 void expert_down_q(const MoeArgs &a, int n_slots, hipStream_t st) {
     if (n_slots <= 0) return;
     if (launch_tk(a, TK_DOWN, n_slots, st, nullptr, nullptr)) return;
-    const int nb = (a.F + 63) / 64, nbp = (nb + 1) & ~1;
-    const int ntok = sk_ntok(a.T, 1, nb);
-    const int threads = 64 * sk_waves(nbp / 2);
-    const size_t lds = (size_t)nb * ntok * 64 + SK_DUMMY;
-    const int grid = n_slots * ((a.D + 15) / 16);
-    if (a.dtype_mask & (1 << 4)) k_expert_down_sk<4><<<grid, threads, lds, st>>>(a, ntok);
-    if (a.dtype_mask & (1 << 3)) k_expert_down_sk<3><<<grid, threads, lds, st>>>(a, ntok);
+    mm_down(a, n_slots, st);
 }
 
 void fgemv(int dtype, const void *W, int rows, int cols, const float *X, int ldx, int T, float *Y, int ldy, hipStream_t st) {
