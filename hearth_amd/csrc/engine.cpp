@@ -869,8 +869,12 @@ void hearth_engine::attn_mla(const Layer &w, int l, int T) {
     at.hd = C; at.cap = cap; at.scale = 1.0f;
     at.g = ma.g;
     at.qo = alat; at.qo_on = 1; at.qo_hm = 1;
-    hxl::attention_scores(at, st);
-    hxl::mla_pe_scores(ma, st);
+    if (rdim == 64) { at.qpe = qb + nope; at.kpe = ma.kp; at.qpe_ld = qh; at.pe_scale = c.attn_scale; }
+    if (!at.qpe || !hxl::scores_many(at, st)) {
+        at.qpe = nullptr;
+        hxl::attention_scores(at, st);
+        hxl::mla_pe_scores(ma, st);
+    }
     hxl::attention_finish(at, st);
     });
     dump("att", l, olat, T, H * C);

@@ -127,6 +127,11 @@ struct AttnArgs {
     const float *rk, *rv, *bq, *bk, *bv, *qn, *kn, *rope;
     float *qout;
     float eps;
+    /* latent attention, or null: the rotated q_pe of (token t, head h) at qpe + (t H + h)
+     * qpe_ld and the RoPE keys [cap][64]; a score is then pe_scale (dot16 + RoPE dot16) */
+    const float *qpe, *kpe;
+    int qpe_ld;
+    float pe_scale;
 };
 
 struct QkvArgs {
@@ -346,6 +351,10 @@ void attention(const AttnArgs &a, hipStream_t st);
 /* the two halves of attention(): scores; softmax + value sum */
 void attention_scores(const AttnArgs &a, hipStream_t st);
 void attention_finish(const AttnArgs &a, hipStream_t st);
+/* the scores (with a.qpe: the latent attention's RoPE term too) and value sums of many rows
+ * (k_attn_many.hip); false: not a shape they take, nothing is launched */
+bool scores_many(const AttnArgs &a, hipStream_t st);
+bool values_many(const AttnArgs &a, hipStream_t st);
 /* attention in the chunked order (64-row chunks folded in order; see k_attn.hip), for
  * head_dim 64 or 128 and grp * head_dim <= 12288 (attention_chunked_ok) */
 bool attention_chunked_ok(int hd, int grp);
