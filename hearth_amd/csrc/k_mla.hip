@@ -71,48 +71,89 @@ __device__ __forceinline__ int seg_bytes(int dt) { return dt == 3 ? 66 : dt == 4
 
 /* mla_qlat (model.c:650-671): ql[t][h][c] = sum_n q[t][h][n] * W_UK[h][n][c], n ascending
  * from 0.0f, with the weight element dequantized as the reference does (d * q). One
- * workgroup per (head, 64 columns): the nope rows' segments of those columns are staged
- * in LDS once (coalesced 2-byte loads), then tiles of QL_TT tokens' q_nope; wave w sums
- * the tokens w, w + 4, ... of a tile, lane l column c0 + l. */
-constexpr int QL_TT = 32;
-__global__ __launch_bounds__(256) void k_mla_qlat(MlaArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t ql_lds[];
+ * workgroup per (head, 64 columns): QL_N nope rows' segments of those columns are staged
+ * in LDS (coalesced 2-byte loads) and dequantized there once; then a wave takes 16 tokens
+ * and 16 CT columns at a time (the four waves are CT token tiles of the 64 columns).
+ *
+ * Every term is a rounded product and an add in order. The products come from
+ * v_mfma_f32_16x16x1_4b_f32 with a zero accumulator (rounded once, exactly fmul): one
+ * register of q and one of W give the 1024 products of 16 tokens, 16 columns and 4 rows n,
+ * so that the adds are all that is left to the vector units. Bound by products and adds for
+ * many tokens, by staging and dequantization for few. Before (a column a lane, the weight
+ * dequantized for every 8 tokens and q read from LDS for every term), now, us a launch, 128
+ * heads of 128 x 512: 301 tokens 668 -> 154, 9 tokens 54 -> 37. */
+constexpr int QL_N = 128;
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+template <int CT>
+__global__ __launch_bounds__(256, 2) void k_mla_qlat(MlaArgs a) {
+    typedef float vct __attribute__((ext_vector_type(CT)));
+    constexpr int CW = 4 / CT;
+    __shared__ __attribute__((aligned(16))) float wf[QL_N * 64];   /* [n][64 columns] */
+    __shared__ __attribute__((aligned(16))) uint8_t raw[QL_N * 256];
     const int dt = a.wuk_dtype, seg = seg_bytes(dt), stride = (seg + 3) & ~3;
     const int ncb = a.C / 64;
     const int h = (int)blockIdx.x / ncb, cb = (int)blockIdx.x % ncb;
-    const int nope = a.nope, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    float *qn = (float *)(ql_lds + (size_t)nope * stride);   /* [QL_TT][nope] */
+    const int tid = threadIdx.x, lane = tid & 63, kg = lane >> 4, lr = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cw = wave % CW, rw = wave / CW;
     const size_t row0 = (size_t)h * (a.nope + a.vd);
     const size_t segoff = dt >= 3 ? (size_t)cb * seg : (size_t)cb * 64 * (dt == 0 ? 4 : 2);
-    {
+    for (int n0 = 0; n0 < a.nope; n0 += QL_N) {
+        const int nn = a.nope - n0 < QL_N ? a.nope - n0 : QL_N;
         const int hw = seg >> 1;   /* 2-byte words per segment */
-        for (int i = tid; i < nope * hw; i += 256) {
+        if (n0) __syncthreads();
+        for (int i = tid; i < nn * hw; i += 256) {
             const int n = i / hw, w = i % hw;
-            const uint16_t *src = (const uint16_t *)(a.wuk + (row0 + n) * a.wuk_rb + segoff);
-            ((uint16_t *)(ql_lds + (size_t)n * stride))[w] = src[w];
-        }
-    }
-    for (int t0 = 0; t0 < a.T; t0 += QL_TT) {
-        const int tn = a.T - t0 < QL_TT ? a.T - t0 : QL_TT;
-        __syncthreads();
-        for (int i = tid; i < tn * nope; i += 256) {
-            const int tt = i / nope, n = i % nope;
-            qn[tt * nope + n] = a.q[((size_t)(t0 + tt) * a.H + h) * a.qh + n];
+            const uint16_t *src = (const uint16_t *)(a.wuk + (row0 + n0 + n) * a.wuk_rb + segoff);
+            ((uint16_t *)(raw + (size_t)n * stride))[w] = src[w];
         }
         __syncthreads();
-        float acc[QL_TT / 4];
+        for (int n = wave; n < nn; n += 4) wf[n * 64 + lane] = deq_elem(raw + (size_t)n * stride, dt, lane);
+        __syncthreads();
+        const int nstep = (nn + 3) / 4;
+        for (int t0 = 16 * rw; t0 < a.T; t0 += 16 * CT) {
+            const int ta = t0 + lr < a.T ? t0 + lr : a.T - 1;
+            const float *qr = a.q + ((size_t)ta * a.H + h) * a.qh + n0;
+            float *dst = a.qlat + ((size_t)(t0 + 4 * kg) * a.H + h) * a.C + cb * 64 + 16 * CT * cw + CT * lr;
+            float acc[CT][4];
 #pragma unroll
-        for (int j = 0; j < QL_TT / 4; j++) acc[j] = 0.0f;
-        for (int n = 0; n < nope; n++) {
-            const float w = deq_elem(ql_lds + (size_t)n * stride, dt, lane);
+            for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int j = 0; j < QL_TT / 4; j++)
-                if (wave + 4 * j < tn) acc[j] = fadd(acc[j], fmul(qn[(wave + 4 * j) * nope + n], w));
+                for (int x = 0; x < CT; x++)
+                    acc[x][r] = n0 && t0 + 4 * kg + r < a.T ? dst[(size_t)r * a.H * a.C + x] : 0.0f;
+            float q[QL_N / 4];   /* lane (kg, lr): element 4 s + kg of token t0 + lr */
+#pragma unroll
+            for (int s = 0; s < QL_N / 4; s++) q[s] = qr[4 * s + kg < nn ? 4 * s + kg : nn - 1];
+#pragma unroll
+            for (int s = 0; s < QL_N / 4; s++) {
+                if (s >= nstep) break;   /* uniform */
+                const vct w = *(const vct *)&wf[(4 * s + kg < nn ? 4 * s + kg : nn - 1) * 64 + 16 * CT * cw + CT * lr];
+                v16f p[CT];
+#pragma unroll
+                for (int x = 0; x < CT; x++) {
+                    const v16f zero = {};
+                    p[x] = __builtin_amdgcn_mfma_f32_16x16x1f32(q[s], w[x], zero, 0, 0, 0);
+                }
+                const int nb = nn - 4 * s;   /* the last step may hold fewer than 4 rows */
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+                    if (b < nb) {   /* uniform */
+#pragma unroll
+                        for (int x = 0; x < CT; x++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) acc[x][r] = fadd(acc[x][r], p[x][4 * b + r]);
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (t0 + 4 * kg + r < a.T) {
+                    vct o;
+#pragma unroll
+                    for (int x = 0; x < CT; x++) o[x] = acc[x][r];
+                    *(vct *)(dst + (size_t)r * a.H * a.C) = o;
+                }
         }
-#pragma unroll
-        for (int j = 0; j < QL_TT / 4; j++)
-            if (wave + 4 * j < tn)
-                a.qlat[((size_t)(t0 + wave + 4 * j) * a.H + h) * a.C + cb * 64 + lane] = acc[j];
     }
 }
 
@@ -190,10 +231,11 @@ void mla_post(const MlaArgs &a, hipStream_t st) {
 }
 
 void mla_qlat(const MlaArgs &a, hipStream_t st) {
-    /* C is a multiple of 128 (checked at open); LDS: nope segments + a token tile */
-    const int dt = a.wuk_dtype, seg = dt == 3 ? 66 : dt == 4 ? 34 : dt == 0 ? 256 : 128;
-    const size_t lds = (size_t)a.nope * ((seg + 3) & ~3) + sizeof(float) * (size_t)QL_TT * a.nope;
-    k_mla_qlat<<<a.H * (a.C / 64), 256, lds, st>>>(a);
+    /* C is a multiple of 128 (checked at open). From four token tiles on every wave has one
+     * of its own; fewer are split by columns */
+    if (a.T > 48) k_mla_qlat<4><<<a.H * (a.C / 64), 256, 0, st>>>(a);
+    else if (a.T > 16) k_mla_qlat<2><<<a.H * (a.C / 64), 256, 0, st>>>(a);
+    else k_mla_qlat<1><<<a.H * (a.C / 64), 256, 0, st>>>(a);
 }
 
 void mla_pe_scores(const MlaArgs &a, hipStream_t st) {
