@@ -448,18 +448,23 @@ __global__ __launch_bounds__(SM_T) void k_attn_softmax(AttnArgs a) {
     }
 }
 
-/* The same softmax with one wave per (token, head) row, for many rows of at most
- * SMW_PER * 64 scores (a tree's or a prefill's): the row's scores and exps stay in the
- * lane's registers, the exps also go to the wave's own LDS slice for the 16 sequential
- * partial sums, and nothing waits on the workgroup: the same operations in the same
- * order as k_attn_softmax, so the same bits. */
+/* The same softmax with one wave per (token, head) row, for many rows of at most 64 PER
+ * scores (a tree's or a prefill's): the row's scores and exps stay in the lane's registers,
+ * the exps also go to the wave's own LDS slice for the 16 sequential partial sums, and
+ * nothing waits on the workgroup: the same operations in the same order as k_attn_softmax,
+ * so the same bits. Four entries a lane at a time, so that their exps and divisions (long
+ * dependent chains of double and single operations) run side by side; PER by the longest
+ * row, since registers and LDS for scores that no row has leave fewer waves in flight.
+ * Bound by the latency of its few waves for short rows, by the traffic of S for long ones
+ * (80 us are 4.9 TB/s). One exp at a time and PER = 48 for all, and this, us a launch of 512
+ * tokens x 32 heads: from empty 47 -> 15, at 2048 91 -> 80; 85 x 32 rows at 2047 20 -> 18. */
 constexpr int SMW_WAVES = 4;
-constexpr int SMW_PER = 48;
-constexpr int SMW_MAX = SMW_PER * 64;
+constexpr int SMW_MAX = 3072;    /* scores of a row */
 constexpr int SMW_ROWS = 1024;   /* rows from which a wave per row beats a workgroup per row */
 
+template <int PER>
 __global__ __launch_bounds__(64 * SMW_WAVES) void k_attn_softmax_w(AttnArgs a) {
-    __shared__ float es_all[SMW_WAVES][SMW_MAX];
+    __shared__ float es_all[SMW_WAVES][64 * PER];
     __shared__ unsigned long long etab[32];
     exp_table_to_lds(etab);
     __syncthreads();
@@ -468,58 +473,81 @@ __global__ __launch_bounds__(64 * SMW_WAVES) void k_attn_softmax_w(AttnArgs a) {
     if (row >= a.T * a.H) return;   /* uniform per wave; no barrier follows */
     const int t = row / a.H, h = row % a.H;
     if (a.g.live && t >= *a.g.live) return;   /* padding token */
-    const int pos0 = *a.g.pos, nr = pos0 + a.g.depth[t] + 1;
+    const int pos0 = *a.g.pos, nr = __builtin_amdgcn_readfirstlane(pos0 + a.g.depth[t] + 1);
     float *s = a.S + ((size_t)t * a.H + h) * a.ldS;
     float *es = es_all[wave];
-    float x[SMW_PER];
+    float x[PER];
     float m = -__builtin_huge_valf();
+    /* every load before the first use; entries past the row repeat its last score (no change
+     * to the maximum) and their exps are never stored or used */
 #pragma unroll
-    for (int u = 0; u < SMW_PER; u++) {
-        const int i = lane + 64 * u;
-        x[u] = i < nr ? s[i] : -__builtin_huge_valf();
+    for (int u0 = 0; u0 < PER; u0 += 4) {
+#pragma unroll
+        for (int u = u0; u < u0 + 4; u++) x[u] = -__builtin_huge_valf();
+        if (64 * u0 < nr) {   /* uniform */
+#pragma unroll
+            for (int u = u0; u < u0 + 4; u++) {
+                const int i = lane + 64 * u;
+                x[u] = s[i < nr ? i : nr - 1];
+            }
+        }
     }
 #pragma unroll
-    for (int u = 0; u < SMW_PER; u++)
+    for (int u = 0; u < PER; u++)
         if (x[u] == x[u]) m = fmaxf(m, x[u]);
     m = wave_max_f32(m);   /* a maximum: any reduction order gives the same value */
     const float s0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x[0])));
     if (s0 != s0) m = s0;
 #pragma unroll
-    for (int u = 0; u < SMW_PER; u++) {
-        if (64 * u < nr) {   /* uniform */
-            const int i = lane + 64 * u;
-            const float e = exp_glibc_f(fadd(x[u], -m), etab);
-            x[u] = e;
-            if (i < nr) es[i] = e;
+    for (int u0 = 0; u0 < PER; u0 += 4)
+        if (64 * u0 < nr) {   /* uniform */
+            float e[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) e[k] = exp_glibc_f(fadd(x[u0 + k], -m), etab);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = lane + 64 * (u0 + k);
+                x[u0 + k] = e[k];
+                if (i < nr) es[i] = e[k];
+            }
         }
-    }
     wave_sync();
     float L = 0.0f;   /* lane < 16: partial of the elements i = lane (mod 16) */
     if (lane < 16) L = sum16_lds(es, nr, lane, L);
     L = tree16(L);
     const float sum = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(L)));
 #pragma unroll
-    for (int u = 0; u < SMW_PER; u++) {
-        const int i = lane + 64 * u;
-        if (64 * u < nr && i < nr) s[i] = fdiv(x[u], sum);
-    }
+    for (int u0 = 0; u0 < PER; u0 += 4)
+        if (64 * u0 < nr) {
+            float y[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) y[k] = fdiv(x[u0 + k], sum);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = lane + 64 * (u0 + k);
+                if (i < nr) s[i] = y[k];
+            }
+        }
 }
 
 /* o[t][h][d] = sum_v p_v * V_v[d], v in order. A workgroup sums up to four heads of
  * one token t in one KV group g, for one 64-wide d chunk: one summing wave per head
  * (lane = column d, one dependent add chain per lane), and eight loader waves.
  *
- * The chain's floor is the add latency (about 8 cycles a row); what a summing wave
- * issues besides the add must fit beside it. So each lane reads its column four rows
- * at a time (one 16-byte LDS read): the loaders store V tiles transposed, as 4-row
- * blocks of [64 columns][4 rows] (+ 4 floats of padding, which puts the 64 lanes of
- * every transposed store in 64 different banks). The p row of the head is read one
- * value per lane per 16 rows and each row's p reaches all lanes by a DPP row broadcast
- * folded into the product (v_mul_f32 with row_newbcast), so p costs no instruction.
+ * The chain's floor is the add latency (4 clocks a row); what a summing wave issues
+ * besides the add comes on top. So each lane reads its column four rows at a time (one
+ * 16-byte LDS read): the loaders store V tiles transposed, as 4-row blocks of [64
+ * columns][4 rows], the columns in an order that gives the 64 lanes of every store 64
+ * words in a row. The p row of the head is read one value per lane per 16 rows and each
+ * row's p reaches all lanes by a DPP row broadcast folded into the product (v_mul_f32 with
+ * row_newbcast). Tiles are published a step before they are summed, so that a tile's first
+ * reads do not wait behind its barrier. Measured, 32 heads at 4095, one token 32.1 -> 29.6
+ * us, 9 tokens 33.1 -> 31.0 (loads of 4 whole rows instead of 16 quarter ones, and the
+ * early first reads); without the sums 14.0 (31.4 before), without the stores 26.7.
  *
  * Loaders: 16-byte buffer loads of V rows into registers, three tiles in flight, then
- * transposed 4-byte stores into one of two V slots; p goes straight from memory into a
- * 4-slot LDS ring (LDS-direct). For a chain geometry row v of every token is cache
+ * transposed 4-byte stores into one of three V slots; p goes straight from memory into a
+ * 5-slot LDS ring (LDS-direct). For a chain geometry row v of every token is cache
  * slot v, so a tile's rows need no lookup, and the buffer's range check turns rows
  * past the cache into zeros; a tree maps each row through the token's ancestor table
  * (clamped to the token's rows). Rows past the token's chain are loaded but never
@@ -527,7 +555,8 @@ __global__ __launch_bounds__(64 * SMW_WAVES) void k_attn_softmax_w(AttnArgs a) {
  * (lgkmcnt(0)); loads in flight stay in flight across it. */
 constexpr int TV_ROWS = 128;            /* rows per tile */
 constexpr int TV_BQ = 260;              /* floats per 4-row block: [64 columns][4 rows] + 4 */
-constexpr int TV_PS = 4;                /* p ring slots */
+constexpr int TV_PS = 4;                /* p ring slots of k_attn_values_w */
+constexpr int TV_PS3 = 5;               /* and of k_attn_values, which publishes a tile earlier */
 constexpr int TV_THREADS = 768;         /* 4 summing + 8 loader waves */
 constexpr int TV_SUM = 4, TV_LOAD = 8;  /* summing waves (one head each), loader waves */
 /* the staging map below: loader wave lw owns tile rows 16 lw .. 16 lw + 15 (lane % 16)
@@ -556,10 +585,19 @@ __device__ __forceinline__ void tv_sum16(float &acc, float P, const float4 (&V)[
     const float q10 = fmul(tv_bc<10>(P), V[2].z), q11 = fmul(tv_bc<11>(P), V[2].w);
     const float q12 = fmul(tv_bc<12>(P), V[3].x), q13 = fmul(tv_bc<13>(P), V[3].y);
     const float q14 = fmul(tv_bc<14>(P), V[3].z), q15 = fmul(tv_bc<15>(P), V[3].w);
+    /* all products, then all adds: k_attn_values_w's 85 x 32 rows at 2047 58 -> 55.8 us a
+     * launch (a lone wave alone on its unit takes 11 clocks a row, 22 with the two in turns) */
+    __builtin_amdgcn_sched_barrier(0);
     acc = fadd(acc, q0); acc = fadd(acc, q1); acc = fadd(acc, q2); acc = fadd(acc, q3);
     acc = fadd(acc, q4); acc = fadd(acc, q5); acc = fadd(acc, q6); acc = fadd(acc, q7);
     acc = fadd(acc, q8); acc = fadd(acc, q9); acc = fadd(acc, q10); acc = fadd(acc, q11);
     acc = fadd(acc, q12); acc = fadd(acc, q13); acc = fadd(acc, q14); acc = fadd(acc, q15);
+}
+
+/* the sum of column `lane` for every lane: place p of a block is column 4 (p % 16) + p / 16 */
+__device__ __forceinline__ float tv_column(float x) {
+    const int lane = threadIdx.x & 63;
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (16 * (lane & 3) + (lane >> 2)), __float_as_int(x)));
 }
 
 /* The extra workgroups of k_attn_values read the ranges pf_p[r][0, pf_n[r]) (the weights
@@ -572,8 +610,8 @@ __device__ void values_read_ahead(const AttnArgs &a, int wg) {
 }
 
 __global__ __launch_bounds__(TV_THREADS) void k_attn_values(AttnArgs a) {
-    __shared__ __attribute__((aligned(16))) float vt[2][(TV_ROWS / 4) * TV_BQ];
-    __shared__ __attribute__((aligned(16))) float pt[TV_PS][4][TV_ROWS];
+    __shared__ __attribute__((aligned(16))) float vt[3][(TV_ROWS / 4) * TV_BQ];
+    __shared__ __attribute__((aligned(16))) float pt[TV_PS3][4][TV_ROWS];
     __shared__ int anc_s[MAX_ANC];
     const int Hkv = a.Hkv, grp = a.H / Hkv, hd = a.hd;
     const int nd = (hd + 63) / 64, qpt = (grp + TV_SUM - 1) / TV_SUM;
@@ -599,31 +637,27 @@ __global__ __launch_bounds__(TV_THREADS) void k_attn_values(AttnArgs a) {
         __syncthreads();
     }
     if (wave >= TV_SUM) {
-        /* loader wave lw: rows 16 lw + lane % 16 of each tile, columns 16 cb + 4 (lane / 16)
-         * .. + 3 for cb = 0..3, and half lw % 2 of head lw / 2's p row */
-        const int lw = wave - TV_SUM, r = lane & 15, cg = lane >> 4, half = lw & 1;
+        /* loader wave lw: rows 16 lw + 4 cb + r of each tile, cb = 0..3 (r = lane / 16),
+         * columns 4 (lane % 16) .. + 3, and half lw % 2 of head lw / 2's p row */
+        const int lw = wave - TV_SUM, r = lane >> 4, half = lw & 1;
         const __amdgpu_buffer_rsrc_t vrs =
             __builtin_amdgcn_make_buffer_rsrc((void *)(a.vc + (size_t)g * a.cap * hd), 0, a.cap * hd * 4, 0x00020000);
-        int coff[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-            const int col = dc * 64 + 16 * cb + 4 * cg;
-            coff[cb] = (col < hd ? col : 0) * 4;
-        }
+        const int col = dc * 64 + 4 * (lane & 15), coff = (col < hd ? col : 0) * 4;
         const int phh = hq * TV_SUM + (lw >> 1);
         const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(a.S + ((size_t)t * a.H + (size_t)g * grp + (phh < grp ? phh : 0)) * a.ldS), 0, a.ldS * 4, 0x00020000);
         const int hd4 = hd * 4, roff = r * hd4;
-        /* word of (row 16 lw + r, column 16 cb + 4 cg + e): bank 16 lw + r + 16 cg + 4 e mod 64 */
-        const int wbase = (4 * lw + (r >> 2)) * TV_BQ + 16 * cg + (r & 3);
+        /* word of (row 16 lw + 4 cb + r, column 4 c + e): block 4 lw + cb, place 16 e + c,
+         * float r: the 64 lanes of a store write 64 words in a row */
+        const int wbase = 4 * lw * TV_BQ + 4 * (lane & 15) + r;
         auto store = [&](int slot, const tv_u4 (&R)[4]) {
             float *w = &vt[slot][wbase];
 #pragma unroll
             for (int cb = 0; cb < 4; cb++) {
-                w[64 * cb + 0] = __uint_as_float(R[cb].x);
-                w[64 * cb + 4] = __uint_as_float(R[cb].y);
-                w[64 * cb + 8] = __uint_as_float(R[cb].z);
-                w[64 * cb + 12] = __uint_as_float(R[cb].w);
+                w[TV_BQ * cb + 0] = __uint_as_float(R[cb].x);
+                w[TV_BQ * cb + 64] = __uint_as_float(R[cb].y);
+                w[TV_BQ * cb + 128] = __uint_as_float(R[cb].z);
+                w[TV_BQ * cb + 192] = __uint_as_float(R[cb].w);
             }
         };
         auto run = [&](auto chain_tag) {
@@ -633,19 +667,21 @@ __global__ __launch_bounds__(TV_THREADS) void k_attn_values(AttnArgs a) {
                 if constexpr (CHAIN) {
                     const int vo = roff + (vb + 16 * lw) * hd4;
 #pragma unroll
-                    for (int cb = 0; cb < 4; cb++) R[cb] = __builtin_amdgcn_raw_buffer_load_b128(vrs, vo + coff[cb], 0, 0);
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (__attribute__((address_space(3))) void *)&pt[i % TV_PS][lw >> 1][64 * half],
+                    for (int cb = 0; cb < 4; cb++) R[cb] = __builtin_amdgcn_raw_buffer_load_b128(vrs, vo + 4 * cb * hd4 + coff, 0, 0);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (__attribute__((address_space(3))) void *)&pt[i % TV_PS3][lw >> 1][64 * half],
                                                              4, (vb + 64 * half + lane) * 4, 0, 0, 0);
                 } else {
-                    int v = vb + 16 * lw + r;
-                    v = v < nr ? v : nr - 1;
-                    const int an = anc_s[v > pos0 ? v - pos0 : 0];
-                    const int srow = v < pos0 ? v : an;
 #pragma unroll
-                    for (int cb = 0; cb < 4; cb++) R[cb] = __builtin_amdgcn_raw_buffer_load_b128(vrs, srow * hd4 + coff[cb], 0, 0);
+                    for (int cb = 0; cb < 4; cb++) {
+                        int v = vb + 16 * lw + 4 * cb + r;
+                        v = v < nr ? v : nr - 1;
+                        const int an = anc_s[v > pos0 ? v - pos0 : 0];
+                        const int srow = v < pos0 ? v : an;
+                        R[cb] = __builtin_amdgcn_raw_buffer_load_b128(vrs, srow * hd4 + coff, 0, 0);
+                    }
                     int vp = vb + 64 * half + lane;
                     vp = vp < nr ? vp : nr - 1;
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (__attribute__((address_space(3))) void *)&pt[i % TV_PS][lw >> 1][64 * half],
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (__attribute__((address_space(3))) void *)&pt[i % TV_PS3][lw >> 1][64 * half],
                                                              4, vp * 4, 0, 0, 0);
                 }
             };
@@ -655,77 +691,73 @@ __global__ __launch_bounds__(TV_THREADS) void k_attn_values(AttnArgs a) {
             load(2, R2);
             HX_WAIT_VMCNT(10);
             store(0, R0);
-            /* step i: tile i is published; tile i + 3 is loaded into the registers tile i came
-             * from; tile i + 1 is stored into the slot tile i - 1 was summed from. The loop
-             * has no exit inside its body, so the compiler keeps the exact load counts. */
+            load(3, R0);
+            HX_WAIT_VMCNT(10);
+            store(1, R1);
+            /* step i: tiles i and i + 1 are published; tile i + 4 is loaded into the registers
+             * tile i + 1 came from; tile i + 2 is stored into the slot tile i - 1 was summed
+             * from. The loop has no exit inside its body, so the compiler keeps the exact
+             * load counts. */
 #define TV_STEP(i_, RL, RW)                                                                 \
             __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0) only */                       \
             __builtin_amdgcn_s_barrier();                                                   \
-            load((i_) + 3, RL);                                                             \
+            load((i_) + 4, RL);                                                             \
             HX_WAIT_VMCNT(10);                                                              \
-            store(((i_) + 1) & 1, RW);
+            store(((i_) + 2) % 3, RW);
             int i = 0;
             for (; i + 3 <= ntiles; i += 3) {
-                TV_STEP(i, R0, R1)
-                TV_STEP(i + 1, R1, R2)
-                TV_STEP(i + 2, R2, R0)
+                TV_STEP(i, R1, R2)
+                TV_STEP(i + 1, R2, R0)
+                TV_STEP(i + 2, R0, R1)
             }
-            /* the last one or two steps load nothing (their tiles would lie past the
-             * rows): the loads of the tiles still to publish are waited for in full. A
-             * step's load count is not a bound here, because the compiler drops register
-             * loads whose values are never used, so a count-based wait could let the
-             * LDS-direct p rows of the tile being published still be in flight */
-#define TV_LAST(i_, RW)                                                                     \
-            __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0) only */                       \
-            __builtin_amdgcn_s_barrier();                                                   \
-            HX_WAIT_VMCNT(0);                                                               \
-            store(((i_) + 1) & 1, RW);
-            if (i < ntiles) {
-                TV_LAST(i, R1)
-                if (i + 1 < ntiles) {
-                    TV_LAST(i + 1, R2)
-                }
+            /* the last one or two steps: their tiles are stored already */
+            for (; i < ntiles; i++) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                __builtin_amdgcn_s_barrier();
             }
-#undef TV_LAST
+            HX_WAIT_VMCNT(0);   /* no LDS write may land after the workgroup ends */
 #undef TV_STEP
         };
         if (chain) run(std::true_type{});
         else run(std::false_type{});
-        HX_WAIT_VMCNT(0);              /* no LDS write may land after the workgroup ends */
     } else {
         const int hh = hq * TV_SUM + wave;
         const bool live = hh < grp;
         const int h = g * grp + (live ? hh : 0);
         float acc = 0.0f;
-        for (int i = 0; i < ntiles; i++) {
-            __syncthreads();
-            const int slot = i & 1, nv = nr - i * TV_ROWS;
-            const float4 *vw = (const float4 *)&vt[slot][lane * 4];
-            if (nv >= TV_ROWS) {
-                const float *pw1 = &pt[i % TV_PS][wave][lane & 15];
-                float4 VA[4], VB[4];
-                float PA, PB;
-                /* one group of 16 rows is read while the previous one is summed; the
-                 * scheduling barriers keep the compiler from sinking the reads */
-#define TV_RD(V_, P_, g_) \
-                _Pragma("unroll") for (int j = 0; j < 4; j++) V_[j] = vw[((g_) * 4 + j) * (TV_BQ / 4)]; P_ = pw1[(g_) * 16];
+        float4 VA[4], VB[4];
+        float PA, PB;
+        /* one group of 16 rows is read while the previous one is summed, a tile's first one
+         * (published a step early) at the end of the tile before it; the scheduling barriers
+         * keep the compiler from sinking the reads */
+#define TV_RD(V_, P_, i_, g_) { \
+                const float4 *vw = (const float4 *)&vt[(i_) % 3][lane * 4]; \
+                _Pragma("unroll") for (int j = 0; j < 4; j++) V_[j] = vw[((g_) * 4 + j) * (TV_BQ / 4)]; \
+                P_ = pt[(i_) % TV_PS3][wave][(lane & 15) + (g_) * 16]; }
 #define TV_SB __builtin_amdgcn_sched_barrier(0);
-                TV_RD(VA, PA, 0)
-                TV_RD(VB, PB, 1) TV_SB tv_sum16(acc, PA, VA); TV_SB
-                TV_RD(VA, PA, 2) TV_SB tv_sum16(acc, PB, VB); TV_SB
-                TV_RD(VB, PB, 3) TV_SB tv_sum16(acc, PA, VA); TV_SB
-                TV_RD(VA, PA, 4) TV_SB tv_sum16(acc, PB, VB); TV_SB
-                TV_RD(VB, PB, 5) TV_SB tv_sum16(acc, PA, VA); TV_SB
-                TV_RD(VA, PA, 6) TV_SB tv_sum16(acc, PB, VB); TV_SB
-                TV_RD(VB, PB, 7) TV_SB tv_sum16(acc, PA, VA); TV_SB
-                tv_sum16(acc, PB, VB);
-#undef TV_SB
-#undef TV_RD
+        for (int i = 0; i < ntiles; i++) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int nv = nr - i * TV_ROWS;
+            if (i == 0) TV_RD(VA, PA, 0, 0)
+            if (nv >= TV_ROWS) {
+                TV_RD(VB, PB, i, 1) TV_SB tv_sum16(acc, PA, VA); TV_SB
+                TV_RD(VA, PA, i, 2) TV_SB tv_sum16(acc, PB, VB); TV_SB
+                TV_RD(VB, PB, i, 3) TV_SB tv_sum16(acc, PA, VA); TV_SB
+                TV_RD(VA, PA, i, 4) TV_SB tv_sum16(acc, PB, VB); TV_SB
+                TV_RD(VB, PB, i, 5) TV_SB tv_sum16(acc, PA, VA); TV_SB
+                TV_RD(VA, PA, i, 6) TV_SB tv_sum16(acc, PB, VB); TV_SB
+                TV_RD(VB, PB, i, 7) TV_SB tv_sum16(acc, PA, VA); TV_SB
+                TV_RD(VA, PA, i + 1, 0) TV_SB tv_sum16(acc, PB, VB); TV_SB
             } else {
-                const float *pv = &pt[i % TV_PS][wave][0];
-                for (int rr = 0; rr < nv; rr++) acc = fadd(acc, fmul(pv[rr], vt[slot][(rr >> 2) * TV_BQ + lane * 4 + (rr & 3)]));
+                const float *pv = &pt[i % TV_PS3][wave][0];
+                for (int rr = 0; rr < nv; rr++) acc = fadd(acc, fmul(pv[rr], vt[i % 3][(rr >> 2) * TV_BQ + lane * 4 + (rr & 3)]));
             }
         }
+#undef TV_SB
+#undef TV_RD
+        acc = tv_column(acc);
         const int d = dc * 64 + lane;
         if (live && d < hd) a.out[(size_t)t * a.H * hd + (size_t)h * hd + d] = acc;
         if (a.qo_on && live) quant_block_wave(acc, a.qo, a.qo_hm ? h * a.T + t : t, a.qo_hm ? dc : h * (hd >> 6) + dc);
@@ -1248,8 +1280,12 @@ void attention_scores(const AttnArgs &a, hipStream_t st) {
 
 void attention_finish(const AttnArgs &a, hipStream_t st) {
     const int grp = a.H / a.Hkv, nd = (a.hd + 63) / 64;
-    if (a.g.nr_max <= SMW_MAX && a.T * a.H >= SMW_ROWS)
-        k_attn_softmax_w<<<(a.T * a.H + SMW_WAVES - 1) / SMW_WAVES, 64 * SMW_WAVES, 0, st>>>(a);
+    if (a.g.nr_max <= SMW_MAX && a.T * a.H >= SMW_ROWS) {
+        const int grid = (a.T * a.H + SMW_WAVES - 1) / SMW_WAVES;
+#define HX_SMW(PER_) if (a.g.nr_max <= 64 * PER_) k_attn_softmax_w<PER_><<<grid, 64 * SMW_WAVES, 0, st>>>(a);
+        HX_SMW(8) else HX_SMW(16) else HX_SMW(24) else HX_SMW(32) else HX_SMW(48)
+#undef HX_SMW
+    }
     else
         k_attn_softmax<<<a.T * a.H, SM_T, 0, st>>>(a);
     const bool wide = (long long)a.T * a.H * nd >= TV_WIDE;
