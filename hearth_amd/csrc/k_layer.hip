@@ -313,26 +313,6 @@ __global__ void k_scale_rows(float *y, int ldy, int T, int n, float s) {
 
 /* ------------------------------------------------------------ routing */
 
-/* a ranks before b: larger value first, NaN last, ties to the lower index */
-__device__ __forceinline__ bool ranks_before(float va, int ia, float vb, int ib) {
-    const bool na = va != va, nb = vb != vb;
-    if (na || nb) return na == nb ? ia < ib : nb;
-    if (va != vb) return va > vb;
-    return ia < ib;
-}
-
-/* wave-wide best (value, index) over candidates; idx < 0 marks "none" */
-__device__ __forceinline__ void wave_best(float &v, int &idx) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(v, off, 64);
-        const int oi = __shfl_xor(idx, off, 64);
-        const bool take = oi >= 0 && (idx < 0 || ranks_before(ov, oi, v, idx));
-        v = take ? ov : v;
-        idx = take ? oi : idx;
-    }
-}
-
 constexpr int ROUTE_EMAX = 1024;
 
 /* the router-logits row token t is routed from: padding tokens (t >= *live) take
@@ -345,107 +325,9 @@ __device__ __forceinline__ int replay_id(const RouteArgs &a, int t, int j) {
     return a.replay[(size_t)(pos % a.replay_rows) * (size_t)(a.n_moe * a.K) + (size_t)a.moe_ord * a.K + j];
 }
 
-/* One wave per token: scores, selection values, group limit, top-K, weights. */
-__global__ __launch_bounds__(64) void k_route_tokens(RouteArgs a) {
-    __shared__ float score[ROUTE_EMAX], sel[ROUTE_EMAX];
-    __shared__ unsigned char taken[ROUTE_EMAX], gkeep[64];
-    __shared__ float gsc[64];
-    const int t = blockIdx.x, lane = threadIdx.x, E = a.E, K = a.K;
-    const float *lg = a.logits + (size_t)route_row(a, t) * E;
-    if (a.score_fn == 0) {
-        /* softmax (quant.c:634-642): m = running max from x[0] (a NaN x[0] makes m NaN) */
-        float m = -__builtin_huge_valf();
-        for (int e = lane; e < E; e += 64) {
-            const float x = lg[e];
-            score[e] = x;
-            if (x == x) m = fmaxf(m, x);
-        }
-        for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-        if (lg[0] != lg[0]) m = lg[0];
-        wave_sync();
-        for (int e = lane; e < E; e += 64) score[e] = exp_glibc_f(fadd(score[e], -m));
-        wave_sync();
-        float L = 0.0f;
-        if (lane < 16)
-            for (int e = lane; e < E; e += 16) L = fadd(L, score[e]);
-        L = tree16(L);
-        const float s = __shfl(L, 0, 64);
-        wave_sync();
-        for (int e = lane; e < E; e += 64) score[e] = fdiv(score[e], s);
-    } else {
-        for (int e = lane; e < E; e += 64) score[e] = fdiv(1.0f, fadd(1.0f, exp_glibc_f(-lg[e])));
-    }
-    wave_sync();
-    for (int e = lane; e < E; e += 64) {
-        sel[e] = a.bias ? fadd(score[e], a.bias[e]) : score[e];
-        taken[e] = 0;
-    }
-    wave_sync();
-    int my_id = -1;
-    if (a.replay) {   /* uniform */
-        if (lane < K) my_id = replay_id(a, t, lane);
-        goto weights;
-    }
-    if (a.n_group > 1) {
-        const int ng = a.n_group, gs = E / ng;
-        for (int g = 0; g < ng; g++) {
-            float v1 = 0.0f, v2 = 0.0f;
-            int i1 = -1, i2 = -1;
-            for (int i = lane; i < gs; i += 64)
-                if (i1 < 0 || ranks_before(sel[g * gs + i], i, v1, i1)) { v1 = sel[g * gs + i]; i1 = i; }
-            wave_best(v1, i1);
-            for (int i = lane; i < gs; i += 64)
-                if (i != i1 && (i2 < 0 || ranks_before(sel[g * gs + i], i, v2, i2))) { v2 = sel[g * gs + i]; i2 = i; }
-            wave_best(v2, i2);
-            if (lane == 0) { gsc[g] = i2 >= 0 ? fadd(v1, v2) : v1; gkeep[g] = 0; }
-        }
-        wave_sync();
-        for (int r = 0; r < a.topk_group; r++) {
-            float v = 0.0f;
-            int bi = -1;
-            for (int g = lane; g < ng; g += 64)
-                if (!gkeep[g] && (bi < 0 || ranks_before(gsc[g], g, v, bi))) { v = gsc[g]; bi = g; }
-            wave_best(v, bi);
-            if (lane == 0) gkeep[bi] = 1;
-            wave_sync();
-        }
-        for (int e = lane; e < E; e += 64)
-            if (!gkeep[e / gs]) sel[e] = 0.0f;
-        wave_sync();
-    }
-    for (int j = 0; j < K; j++) {
-        float v = 0.0f;
-        int bi = -1;
-        for (int e = lane; e < E; e += 64)
-            if (!taken[e] && (bi < 0 || ranks_before(sel[e], e, v, bi))) { v = sel[e]; bi = e; }
-        wave_best(v, bi);
-        if (lane == 0) taken[bi] = 1;
-        if (lane == j) my_id = bi;
-        wave_sync();
-    }
-weights:
-    /* weights: w_j = score[id_j]; norm_topk: w_j / (sum_j w_j + 1e-20f), sum in rank order */
-    float w = lane < K ? score[my_id] : 0.0f;
-    if (a.norm_topk) {
-        float s = 0.0f;
-        for (int j = 0; j < K; j++) {
-            const int idj = __shfl(my_id, j, 64);
-            s = fadd(s, score[idj]);
-        }
-        const float den = fadd(s, 1e-20f);
-        w = fdiv(w, den);
-    }
-    w = fmul(w, a.routed_scale);
-    if (lane < K) {
-        a.ids[(size_t)t * K + lane] = my_id;
-        a.wts[(size_t)t * K + lane] = w;
-        if (a.route_out) a.route_out[((size_t)t * a.n_moe + a.moe_ord) * K + lane] = my_id;
-    }
-}
-
 /* Selection key of (value v, expert e): a larger key ranks first, and the order is
- * ranks_before's: larger value first (-0 equals +0), NaN after every number, ties to
- * the lower index. */
+ * the reference's: larger value first (-0 equals +0), NaN after every number, ties to the
+ * lower index. No key is 0. */
 __device__ __forceinline__ uint32_t order_key(float v) {
     /* a larger value has a larger key (-0 equals +0); NaN has key 0, below every number */
     if (v != v) return 0u;
@@ -455,6 +337,116 @@ __device__ __forceinline__ uint32_t order_key(float v) {
 
 __device__ __forceinline__ unsigned long long rank_key(float v, int e) {
     return ((unsigned long long)order_key(v) << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)e);
+}
+
+/* One wave per token: scores, selection values, group limit, top-K, weights. Lane l holds
+ * the selection keys of experts l, l + 64, ...; each choice is a wave maximum of keys (DPP
+ * steps on the vector units). Bound by that chain of maxima; with values and indices
+ * exchanged through LDS for every choice 37.6 us a launch of 256 experts in 8 groups, now
+ * 14.3. */
+template <int PER>   /* at most 64 PER experts */
+__global__ __launch_bounds__(64) void k_route_tokens(RouteArgs a) {
+    __shared__ float score[64 * PER];
+    __shared__ unsigned long long etab[32];
+    const int t = blockIdx.x, lane = threadIdx.x, E = a.E, K = a.K;
+    const float *lg = a.logits + (size_t)route_row(a, t) * E;
+    exp_table_to_lds(etab);
+    wave_sync();
+    if (a.score_fn == 0) {
+        /* softmax (quant.c:634-642): m = running max from x[0] (a NaN x[0] makes m NaN) */
+        float m = -__builtin_huge_valf();
+        for (int e = lane; e < E; e += 64) {
+            const float x = lg[e];
+            score[e] = x;
+            if (x == x) m = fmaxf(m, x);
+        }
+        m = wave_max_f32(m);
+        if (lg[0] != lg[0]) m = lg[0];
+        wave_sync();
+        for (int e = lane; e < E; e += 64) score[e] = exp_glibc_f(fadd(score[e], -m), etab);
+        wave_sync();
+        float L = 0.0f;
+        if (lane < 16)
+            for (int e = lane; e < E; e += 16) L = fadd(L, score[e]);
+        L = tree16(L);
+        const float s = __shfl(L, 0, 64);
+        wave_sync();
+        for (int e = lane; e < E; e += 64) score[e] = fdiv(score[e], s);
+    } else {
+        for (int e = lane; e < E; e += 64) score[e] = fdiv(1.0f, fadd(1.0f, exp_glibc_f(-lg[e], etab)));
+    }
+    wave_sync();
+    auto sel = [&](int e) { return a.bias ? fadd(score[e], a.bias[e]) : score[e]; };
+    int my_id = -1;
+    if (a.replay) {   /* uniform */
+        if (lane < K) my_id = replay_id(a, t, lane);
+    } else {
+        unsigned long long key[PER];   /* 0: no expert, or taken */
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            key[u] = 0ull;
+            if (64 * u < E) {   /* uniform */
+                const int e = lane + 64 * u;
+                if (e < E) key[u] = rank_key(sel(e), e);
+            }
+        }
+        auto index = [](unsigned long long k) { return (int)(0xFFFFFFFFu - (uint32_t)k); };
+        if (a.n_group > 1) {
+            const int ng = a.n_group, gs = E / ng;
+            unsigned long long gkey = 0ull;   /* lane g: of group g's score, the sum of its best two */
+            for (int g = 0; g < ng; g++) {
+                unsigned long long k1 = 0ull, k2 = 0ull;
+#pragma unroll
+                for (int u = 0; u < PER; u++)
+                    if (64 * u < E) {
+                        const int e = lane + 64 * u;
+                        if (e >= g * gs && e < (g + 1) * gs) {
+                            k2 = key[u] > k1 ? k1 : key[u] > k2 ? key[u] : k2;
+                            k1 = key[u] > k1 ? key[u] : k1;
+                        }
+                    }
+                const unsigned long long m1 = wave_max_u64(k1), m2 = wave_max_u64(k1 == m1 ? k2 : k1);
+                const float v1 = sel(index(m1));
+                const float gs2 = m2 ? fadd(v1, sel(index(m2))) : v1;
+                if (lane == g) gkey = rank_key(gs2, g);
+            }
+            unsigned long long keep = 0ull;
+            for (int r = 0; r < a.topk_group; r++) {
+                const int g = index(wave_max_u64(gkey));
+                keep |= 1ull << g;
+                if (lane == g) gkey = 0ull;
+            }
+#pragma unroll
+            for (int u = 0; u < PER; u++)
+                if (64 * u < E) {
+                    const int e = lane + 64 * u;
+                    if (e < E && !(keep >> (e / gs) & 1)) key[u] = rank_key(0.0f, e);
+                }
+        }
+        for (int j = 0; j < K; j++) {
+            unsigned long long k = 0ull;
+#pragma unroll
+            for (int u = 0; u < PER; u++) k = key[u] > k ? key[u] : k;
+            const unsigned long long m = wave_max_u64(k);
+#pragma unroll
+            for (int u = 0; u < PER; u++) key[u] = key[u] == m ? 0ull : key[u];
+            if (lane == j) my_id = index(m);
+        }
+    }
+    /* weights: w_j = score[id_j]; norm_topk: w_j / (sum_j w_j + 1e-20f), sum in rank order */
+    float w = lane < K ? score[my_id] : 0.0f;
+    if (a.norm_topk) {
+        float s = 0.0f;
+        for (int j = 0; j < K; j++) s = fadd(s, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j)));
+        const float den = fadd(s, 1e-20f);
+        w = fdiv(w, den);
+    }
+    w = fmul(w, a.routed_scale);
+    if (lane < K) {
+        a.ids[(size_t)t * K + lane] = my_id;
+        a.wts[(size_t)t * K + lane] = w;
+        if (a.route_out) a.route_out[((size_t)t * a.n_moe + a.moe_ord) * K + lane] = my_id;
+    }
 }
 
 /* Ungrouped routing (n_group <= 1), one workgroup per token: scores, selection values,
@@ -653,7 +645,7 @@ __global__ __launch_bounds__(1024) void k_route_bucket(RouteArgs a) {
  * workgroup. Wave t routes token t: scores and weights as k_route_rank; the K experts by
  * K rounds of a wave maximum of the 32-bit order keys of the selection values, the winner
  * being the lowest expert index that holds the maximum (ballots in index order), which is
- * ranks_before's order. Each choice sets the token's bit in its expert's token mask, so
+ * the reference's order (ranks_before). Each choice sets the token's bit in its expert's token mask, so
  * the bucketing needs no counting pass: an expert's pair count is the popcount of its
  * mask, and a pair's place among its expert's pairs (tokens ascending, model.c:1030-1035)
  * the popcount of the mask bits below its token (a token's K experts are distinct:
@@ -1138,7 +1130,8 @@ void route(const RouteArgs &a, hipStream_t st) {
         k_route_small<<<1, 1024, 0, st>>>(a);
         return;
     }
-    if (a.n_group > 1) k_route_tokens<<<a.T, 64, 0, st>>>(a);
+    if (a.n_group > 1 && a.E <= 256) k_route_tokens<4><<<a.T, 64, 0, st>>>(a);
+    else if (a.n_group > 1) k_route_tokens<ROUTE_EMAX / 64><<<a.T, 64, 0, st>>>(a);
     else k_route_rank<<<a.T, 256, 0, st>>>(a);
     k_route_bucket<<<1, 1024, 0, st>>>(a);
 }
