@@ -12,6 +12,7 @@
 #include "hx_device.h"
 #include "hx_launch.h"
 #include <hip/hip_ext.h>
+#include <type_traits>
 
 using namespace hxd;
 
@@ -87,9 +88,13 @@ constexpr int SK_MAXP = 4;      /* block pairs per wave */
 constexpr int TK_WAVES_GATEUP = 8;   /* waves per workgroup of k_expert_tk: gate/up (token blocks staged once for 8 waves) */
 constexpr int TK_WAVES_DOWN = 4;     /* and down (more, smaller workgroups over the shorter rows) */
 constexpr size_t TK_LDS_MAX = 65536;
+constexpr int TK_MIXED_T = 4;        /* k_expert_tk for experts of both dtypes: tokens at most */
 constexpr int TK_CHUNK_ROWS = 128;   /* rows of a slot kept on one XCD (two 128-byte scale lines) */
 constexpr int SK_LDS = 65536;   /* bytes of terms per workgroup */
 constexpr int SK_DUMMY = 1024;  /* LDS after the terms: stores of padding token columns */
+/* the split-K kernels of the experts: tokens at most, and the workgroups of the chunked
+ * kernels from which those are the faster ones (few_workgroups) */
+constexpr int SK_T = 4, SK_WGS_GATEUP = 96, SK_WGS_DOWN = 256;
 
 /* Terms of pairs [p0, p1) of row tile rt of the NM matrices ms (same dtype DT and
  * blocks, one shared activation) for tokens t0 .. t0 + 15 (token t's activation row
@@ -535,38 +540,123 @@ __global__ __launch_bounds__(512) void k_expert_tk(MoeArgs a, int rpw, int S, in
     }
 }
 
-/* launches k_expert_tk for experts of at most 16 tokens and one dtype; false when the
- * shape does not fit (the caller uses the general kernels) */
+/* k_expert_tk of one dtype: workgroup shape, or W = 0 when it does not fit */
+struct TkPlan {
+    int rpw, S, W;
+    size_t lds;
+    bool qf;   /* gate/up: its workgroups can quantize the SwiGLU rows */
+};
+
+TkPlan tk_plan(const MoeArgs &a, bool down, int dt) {
+    const int K = down ? a.F : a.D;
+    const int nb = (K + 63) / 64, nbp = (nb + 1) & ~1, npair = nbp / 2;
+    const int NP = dt == 4 ? TkCfg<4>::NP : TkCfg<3>::NP, NM = down ? 1 : 2;
+    const int waves = down ? TK_WAVES_DOWN : TK_WAVES_GATEUP;
+    TkPlan p;
+    p.S = (npair + NP - 1) / NP;
+    p.rpw = p.S < waves ? waves / p.S : 1;
+    p.W = p.rpw * p.S;
+    /* gate/up workgroups of 4 or 8 row tiles cover whole blocks of the SwiGLU rows: they
+     * quantize them too (F a multiple of 128, so the blocks need no padding block) */
+    p.qf = !down && a.mid.q && a.F % 128 == 0 && (p.rpw == 4 || p.rpw == 8) && a.mid.nbp == a.F / 64;
+    p.lds = tk_lds_bytes(nbp, NM, NP, p.rpw, p.S, p.qf);
+    if (p.W > 8 || p.lds > TK_LDS_MAX) p.W = 0;
+    return p;
+}
+
+/* launches k_expert_tk for experts of at most 16 tokens; 0 when the shape does not fit (the
+ * caller uses another kernel), 2 when the launch also quantized the SwiGLU rows. Experts of
+ * both dtypes: a launch each, whose workgroups leave the other's slots alone, and for few
+ * tokens only. Both products of 8 of 128 such experts a token (2048 x 768), these and the
+ * chunked kernels, us: one token 32.5 / 39.6, four 43.1 / 45.5, six 52.4 / 49.6, 16 116 / 60. */
 int launch_tk(const MoeArgs &a, int mode, int n_slots, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     const bool down = mode == TK_DOWN;
     const bool q4 = a.dtype_mask & (1 << 4), q8 = a.dtype_mask & (1 << 3);
-    if (a.T > 16 || q4 == q8) return 0;
-    const int K = down ? a.F : a.D, rows = down ? a.D : a.F;
-    const int nb = (K + 63) / 64, nbp = (nb + 1) & ~1, npair = nbp / 2;
-    const int NP = q4 ? TkCfg<4>::NP : TkCfg<3>::NP, NM = down ? 1 : 2;
-    const int S = (npair + NP - 1) / NP;
-    const int waves = down ? TK_WAVES_DOWN : TK_WAVES_GATEUP;
-    const int rpw = S < waves ? waves / S : 1, W = rpw * S;
-    /* gate/up workgroups of 4 or 8 row tiles cover whole blocks of the SwiGLU rows: they
-     * quantize them too (F a multiple of 128, so the blocks need no padding block) */
-    const bool qf = mode == TK_GATEUP && a.mid.q && a.F % 128 == 0 && (rpw == 4 || rpw == 8) && a.mid.nbp == a.F / 64;
-    const size_t lds = tk_lds_bytes(nbp, NM, NP, rpw, S, qf);
-    if (W > 8 || lds > TK_LDS_MAX) return 0;
-    const int tpw = ((rows + 15) / 16 + rpw - 1) / rpw;
+    if (a.T > (q4 && q8 ? TK_MIXED_T : 16)) return 0;
+    const TkPlan p4 = tk_plan(a, down, 4), p8 = tk_plan(a, down, 3);
+    if ((q4 && !p4.W) || (q8 && !p8.W)) return 0;
+    const bool qf = mode == TK_GATEUP && (!q4 || p4.qf) && (!q8 || p8.qf);
+    const int rows = down ? a.D : a.F;
     /* gate/up: a workgroup per group of 4 tokens; down: one runs all of its slot's groups */
     const int gmax = down ? 1 : (a.T + 3) / 4;   /* tokens per slot <= T */
-    const int ch = tk_chunk(rpw);
-    const int chunks = n_slots * ((tpw + ch - 1) / ch);
-    const dim3 grid(8 * ((chunks + 7) / 8) * ch * gmax), block(64 * W);
-#define TK_LAUNCH(DT_, MODE_) \
-    hipExtLaunchKernelGGL(k_expert_tk<DT_, MODE_>, grid, block, (uint32_t)lds, st, ev0, ev1, 0u, a, rpw, S, gmax, n_slots)
-    if (mode == TK_GATEUP) {
-        if (qf) { if (q4) TK_LAUNCH(4, TK_GATEUP_Q); else TK_LAUNCH(3, TK_GATEUP_Q); }
-        else { if (q4) TK_LAUNCH(4, TK_GATEUP); else TK_LAUNCH(3, TK_GATEUP); }
-    }
-    if (mode == TK_DOWN) { if (q4) TK_LAUNCH(4, TK_DOWN); else TK_LAUNCH(3, TK_DOWN); }
+    auto run = [&](auto dt, const TkPlan &p, hipEvent_t e0, hipEvent_t e1) {
+        constexpr int DT = decltype(dt)::value;
+        const int tpw = ((rows + 15) / 16 + p.rpw - 1) / p.rpw;
+        const int ch = tk_chunk(p.rpw);
+        const int chunks = n_slots * ((tpw + ch - 1) / ch);
+        const dim3 grid(8 * ((chunks + 7) / 8) * ch * gmax), block(64 * p.W);
+#define TK_LAUNCH(MODE_) \
+    hipExtLaunchKernelGGL(k_expert_tk<DT, MODE_>, grid, block, (uint32_t)p.lds, st, e0, e1, 0u, a, p.rpw, p.S, gmax, n_slots)
+        if (down) TK_LAUNCH(TK_DOWN);
+        else if (qf) TK_LAUNCH(TK_GATEUP_Q);
+        else TK_LAUNCH(TK_GATEUP);
 #undef TK_LAUNCH
+    };
+    if (q4) run(std::integral_constant<int, 4>{}, p4, ev0, q8 ? nullptr : ev1);
+    if (q8) run(std::integral_constant<int, 3>{}, p8, q4 ? nullptr : ev0, ev1);
     return qf ? 2 : 1;
+}
+
+/* Split-K products of experts whose K does not fit k_expert_tk, for the few tokens at which
+ * the chunked kernels (k_mm.hip) have too few workgroups: those walk K in order, so that a
+ * launch takes the latency of its K however little work it has, while here each wave loads
+ * its part of K at once. Bound by the weight bytes in flight. Measured, these / the chunked
+ * ones, us a launch (in brackets the chunked workgroups of a dtype): down of K = 6144 to 2048
+ * rows, two Q4 experts a token, 1 token (64) 10.3 / 18.2, 3 (192) 15.4 / 19.2, 4 (256) 22.0 /
+ * 19.3, Q8 1 token 11.2 / 20.1; gate/up and the quantization of its rows, 768 rows of K =
+ * 8192, 1 token (48) 21.8 / 39.9, 2 (96) 35.8 / 40.6, of K = 6144, 1 token (96) 32.8 / 32.4. */
+template <int DT>
+__global__ __launch_bounds__(512) void k_expert_gateup_sk(MoeArgs a, int ntok) {
+    extern __shared__ float P[];
+    const int ntile = a.F / 16;
+    const int u = (int)blockIdx.x / ntile, rt = (int)blockIdx.x % ntile;
+    if (u >= *a.n_active) return;   /* uniform */
+    const SlotDesc &sd = a.desc[u];
+    const int n = sd.n, p0 = sd.p0;
+    const QMat ms[2] = {sd.w.gate, sd.w.up};
+    if (ms[0].dtype != DT) return;   /* the launcher runs one instantiation per dtype */
+    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x;
+    int q0, q1;
+    wave_pairs(ms[0].nbp >> 1, W, wave, q0, q1);
+    const int pstride = ms[0].nb * ntok * 16;
+    const int *ptok = a.pair_tok + p0;
+    for (int t0 = 0; t0 < n; t0 += ntok) {
+        tile_terms<DT, 2>(ms, rt, a.x, t0, n, ntok, [ptok](int t) { return ptok[t]; }, q0, q1, P, pstride);
+        __syncthreads();
+        const int nc = n - t0 < ntok ? n - t0 : ntok;
+        for (int f = tid; f < nc * 16; f += blockDim.x) {
+            const float gv = canon(fold_terms(P, ms[0].nb, ntok, f));
+            const float uv = canon(fold_terms(P + pstride, ms[0].nb, ntok, f));
+            const float sg = fdiv(gv, fadd(1.0f, exp_glibc_f(-gv)));
+            a.midf[(size_t)(p0 + t0 + (f >> 4)) * a.F + rt * 16 + (f & 15)] = fmul(sg, uv);
+        }
+        __syncthreads();
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(512) void k_expert_down_sk(MoeArgs a, int ntok) {
+    extern __shared__ float P[];
+    const int ntile = (a.D + 15) / 16;
+    const int u = (int)blockIdx.x / ntile, rt = (int)blockIdx.x % ntile;
+    if (u >= *a.n_active) return;   /* uniform */
+    const SlotDesc &sd = a.desc[u];
+    const int n = sd.n, p0 = sd.p0;
+    const QMat m = sd.w.down;
+    if (m.dtype != DT) return;
+    const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, tid = threadIdx.x;
+    int q0, q1;
+    wave_pairs(m.nbp >> 1, W, wave, q0, q1);
+    for (int t0 = 0; t0 < n; t0 += ntok) {
+        tile_terms<DT, 1>(&m, rt, a.mid, t0, n, ntok, [p0](int t) { return p0 + t; }, q0, q1, P, 0);
+        __syncthreads();
+        const int nc = n - t0 < ntok ? n - t0 : ntok;
+        for (int f = tid; f < nc * 16; f += blockDim.x) {
+            const int row = rt * 16 + (f & 15);
+            if (row < m.rows) a.Y[(size_t)(p0 + t0 + (f >> 4)) * a.D + row] = canon(fold_terms(P, m.nb, ntok, f));
+        }
+        __syncthreads();
+    }
 }
 
 /* ------------------------------------------------------------ float matrices (dot16) */
@@ -736,16 +826,30 @@ void gemm(const GemmArgs &in, hipStream_t st) {
     else mm_dense(in, st);
 }
 
+/* few tokens whose chunked product (k_mm.hip) would be fewer than `least` workgroups of each
+ * dtype: the split-K kernels of the experts */
+static bool few_workgroups(const MoeArgs &a, int n_slots, int row_groups, int least) {
+    const bool both = (a.dtype_mask & (1 << 4)) && (a.dtype_mask & (1 << 3));
+    return a.T <= SK_T && n_slots * row_groups < (both ? 2 : 1) * least;
+}
+
 /* gate/up; true when the launch also quantized the SwiGLU rows into a.mid. ev0 / ev1
  * (optional) are recorded by the dispatch itself: ev0 at the start of the first launch, ev1
  * at the end of the last. */
 bool expert_gateup(const MoeArgs &a, int n_slots, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     if (n_slots <= 0) return false;
-    /* at most 16 tokens per expert, one dtype, token blocks within its LDS: the split-K
-     * kernel (one term per lane); else the chunked one */
     if (const int r = launch_tk(a, TK_GATEUP, n_slots, st, ev0, ev1)) return r == 2;
-    mm_gateup(a, n_slots, st, ev0, ev1);
-    return true;
+    if (!few_workgroups(a, n_slots, a.F / 64, SK_WGS_GATEUP)) {
+        mm_gateup(a, n_slots, st, ev0, ev1);
+        return true;
+    }
+    const int nb = (a.D + 63) / 64, ntok = sk_ntok(a.T, 2, nb), threads = 64 * sk_waves((nb + 1) / 2);
+    const uint32_t lds = (uint32_t)2 * nb * ntok * 64 + SK_DUMMY;
+    const dim3 grid(n_slots * (a.F / 16));
+    const bool q4 = a.dtype_mask & (1 << 4), q8 = a.dtype_mask & (1 << 3);
+    if (q4) hipExtLaunchKernelGGL(k_expert_gateup_sk<4>, grid, dim3(threads), lds, st, ev0, q8 ? nullptr : ev1, 0u, a, ntok);
+    if (q8) hipExtLaunchKernelGGL(k_expert_gateup_sk<3>, grid, dim3(threads), lds, st, q4 ? nullptr : ev0, ev1, 0u, a, ntok);
+    return false;
 }
 
 /* NUMERICS §2 of the SwiGLU rows of all T * top_k pairs (unless the gate/up launch did
@@ -759,7 +863,15 @@ void expert_down(const MoeArgs &a, int n_slots, hipStream_t st, bool mid_done) {
 void expert_down_q(const MoeArgs &a, int n_slots, hipStream_t st) {
     if (n_slots <= 0) return;
     if (launch_tk(a, TK_DOWN, n_slots, st, nullptr, nullptr)) return;
-    mm_down(a, n_slots, st);
+    if (a.head_slots || !few_workgroups(a, n_slots, (a.D + 63) / 64, SK_WGS_DOWN)) {
+        mm_down(a, n_slots, st);
+        return;
+    }
+    const int nb = a.F / 64, ntok = sk_ntok(a.T, 1, nb), threads = 64 * sk_waves((nb + 1) / 2);
+    const uint32_t lds = (uint32_t)nb * ntok * 64 + SK_DUMMY;
+    const dim3 grid(n_slots * ((a.D + 15) / 16));
+    if (a.dtype_mask & (1 << 4)) k_expert_down_sk<4><<<grid, threads, lds, st>>>(a, ntok);
+    if (a.dtype_mask & (1 << 3)) k_expert_down_sk<3><<<grid, threads, lds, st>>>(a, ntok);
 }
 
 void fgemv(int dtype, const void *W, int rows, int cols, const float *X, int ldx, int T, float *Y, int ldy, hipStream_t st) {
