@@ -112,15 +112,7 @@ struct Layer {
     int dtype_mask = 0;             /* bit dt set when some expert has dtype dt */
 };
 
-
 } // namespace
-
-/* rows from which the value kernel reads the next products' weights ahead: its sums last as
- * long as the reads only from about 1500 rows on. 8 layers of the 2048-wide model, with and
- * without: 9 tokens at 100 917 / 841 us, at 500 948 / 895, at 1500 996 / 999, at 4095 1223 /
- * 1230; one token at 500 721 / 672, at 4095 880 / 880; 48 layers of 9 tokens at 4095 with it
- * 6.52 ms against 6.58 */
-constexpr int READ_AHEAD_ROWS = 1536;
 
 struct hearth_engine {
     hearth_options opt{};
@@ -958,9 +950,10 @@ void hearth_engine::forward(int T, bool want_logits, int /*logit_rows_from*/) {
             at.g.depth = depth; at.g.anc = anc; at.g.anc_ld = B; at.g.pos = d_pos; at.g.nr_max = nr_max(T); at.g.chain = geom_chain;
             at.g.live = route_live;
             at.qo = aatt; at.qo_on = w.o.quant && hd % 64 == 0;
-            if (read_ahead > 0 && at.g.nr_max >= READ_AHEAD_ROWS) {
+            if (read_ahead > 0 && at.g.nr_max > hxd::read_ahead_pos(T)) {
                 /* the value kernel reads ahead this layer's output projection and router and
-                 * the next layer's QKV weights */
+                 * the next layer's QKV weights (once the position, which a captured step's bound
+                 * lies above, has come that far) */
                 int r = 0;
                 auto add = [&](const DMat &m) {
                     if (!m.quant || r + 2 > hxd::AF_NR) return;

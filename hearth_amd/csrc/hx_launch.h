@@ -100,6 +100,13 @@ struct TokGeom {
 };
 
 constexpr int AF_NR = 10;     /* read-ahead ranges of the value kernel */
+/* position from which the value kernel of T tokens reads the next products' weights ahead:
+ * only then do its sums last as long as the reads, and later for more tokens, whose scores and
+ * softmax take their time too. 8 layers of the 2048-wide model in an engine of 8192 positions,
+ * with / without, us: one token at 1000 717 / 694, 1100 715 / 714, 1200 712 / 714, 1500 724 /
+ * 736, 4095 868 / 879; 2 tokens at 1300 755 / 748, 1400 755 / 755, 1500 759 / 764; 9 tokens at
+ * 1000 922 / 895, 1300 933 / 919, 1500 959 / 958, 1700 947 / 951, 4095 1174 / 1184 */
+constexpr __host__ __device__ int read_ahead_pos(int T) { return T > 1 ? 1472 : 1152; }
 
 struct AttnArgs {
     const float *q;           /* [T][H][hd] after qk-norm and RoPE */

@@ -603,8 +603,10 @@ __device__ __forceinline__ float tv_column(float x) {
 /* The extra workgroups of k_attn_values read the ranges pf_p[r][0, pf_n[r]) (the weights
  * of the products after the attention, so that those find them in the memory-side cache
  * instead of HBM). The value kernel is a chain of latencies on a part of the compute
- * units; these reads run beside it on the others. */
+ * units; these reads run beside it on the others. Decided here and not by the host, whose
+ * bound of a captured step's rows lies up to 1023 rows above the position. */
 __device__ void values_read_ahead(const AttnArgs &a, int wg) {
+    if (*a.g.pos < read_ahead_pos(a.T)) return;
     for (int r = 0; r < AF_NR; r++)
         if (a.pf_p[r]) read_lines_ahead(a.pf_p[r], a.pf_n[r], wg, a.pf_wgs);
 }
@@ -1302,8 +1304,13 @@ void attention_finish(const AttnArgs &a, hipStream_t st) {
      * heads: 27.08 against 27.50 with two heads per wave on 8 waves, 28.4 with 12) */
     if (wide && grp >= 8) HX_TV(8, 4, 1, 64)
 #undef HX_TV
-    const int qpt = (grp + TV_SUM - 1) / TV_SUM;
-    k_attn_values<<<a.T * qpt * a.Hkv * nd + a.pf_wgs, TV_THREADS, 0, st>>>(a);
+    const int qpt = (grp + TV_SUM - 1) / TV_SUM, nmain = a.T * qpt * a.Hkv * nd;
+    /* a workgroup fills one of the 256 compute units: reads ahead only while the sums' last
+     * round leaves some free (16 tokens of 32 heads in groups of 8 fill them all: 8 layers, with
+     * / without, us: at 1400 1404 / 1300, at 4095 1726 / 1623, at 7000 2028 / 1925; 9 tokens of
+     * 16 single heads take 288: at 4095 1639 / 1653) */
+    const int ahead = nmain % 256 ? a.pf_wgs : 0;
+    k_attn_values<<<nmain + ahead, TV_THREADS, 0, st>>>(a);
 }
 
 /* the items of a block (grp / rw per token) must fit the block's waves: k_attn_chunk
