@@ -359,9 +359,10 @@ void attention(const AttnArgs &a, hipStream_t st);
 void attention_scores(const AttnArgs &a, hipStream_t st);
 void attention_finish(const AttnArgs &a, hipStream_t st);
 /* the scores (with a.qpe: the latent attention's RoPE term too) and value sums of many rows
- * (k_attn_many.hip); false: not a shape they take, nothing is launched */
+ * (k_attn_many.hip); false: not a shape they take or (values) not expected to take less than
+ * other_ns, nothing is launched */
 bool scores_many(const AttnArgs &a, hipStream_t st);
-bool values_many(const AttnArgs &a, hipStream_t st);
+bool values_many(const AttnArgs &a, double other_ns, hipStream_t st);
 /* attention in the chunked order (64-row chunks folded in order; see k_attn.hip), for
  * head_dim 64 or 128 and grp * head_dim <= 12288 (attention_chunked_ok) */
 bool attention_chunked_ok(int hd, int grp);

@@ -1290,8 +1290,14 @@ void attention_finish(const AttnArgs &a, hipStream_t st) {
     }
     else
         k_attn_softmax<<<a.T * a.H, SM_T, 0, st>>>(a);
-    const bool wide = (long long)a.T * a.H * nd >= TV_WIDE;
-    if (values_many(a, st)) return;
+    const bool wide = (long long)a.T * a.H * nd >= TV_WIDE && grp >= 8;
+    /* what the kernels below take, in ns: 256 workgroups of theirs 7.4 a row (two a unit) and
+     * their prologue, and never less than one round. Within 10% of 13 shapes of 1 to 64 heads
+     * a group and 64 to 512 columns, 17 to 512 tokens at 0, 1000 and 4000 */
+    const int per = wide ? 8 : TV_SUM;
+    const double rounds = (double)a.T * ((grp + per - 1) / per) * a.Hkv * nd / 256;
+    const double rows = a.g.nr_max - (a.g.chain ? a.T / 2.0 : a.T);
+    if (values_many(a, std::max(rounds, wide ? 1.35 : 2.0) * ((wide ? 2300 : 3500) + 7.4 * rows), st)) return;
 #define HX_TV(NS_, NL_, R_, ROWS_)                                                                     \
     {                                                                                                  \
         const int qpt = (grp + NS_ * R_ - 1) / (NS_ * R_);                                             \
@@ -1302,7 +1308,7 @@ void attention_finish(const AttnArgs &a, hipStream_t st) {
      * tokens: 16.91 ms per step against 17.04 with two heads per wave on 4 waves, 17.97
      * with 8 loader waves and 128-row tiles, 19.91 with four heads per wave; MLA's 128
      * heads: 27.08 against 27.50 with two heads per wave on 8 waves, 28.4 with 12) */
-    if (wide && grp >= 8) HX_TV(8, 4, 1, 64)
+    if (wide) HX_TV(8, 4, 1, 64)
 #undef HX_TV
     const int qpt = (grp + TV_SUM - 1) / TV_SUM, nmain = a.T * qpt * a.Hkv * nd;
     /* a workgroup fills one of the 256 compute units: reads ahead only while the sums' last

@@ -464,17 +464,35 @@ bool scores_many(const AttnArgs &a, hipStream_t st) {
 #undef HX_SM
 }
 
-bool values_many(const AttnArgs &a, hipStream_t st) {
+/* ns of k_values_many<CT>: rounds of the workgroups that fit the chip at once (two a compute
+ * unit), the longest rows first. A row is 64 / 42 ns (CT = 4 / 2) while a unit has one of them
+ * and 79 / 49 with two; a tree's steps over its own nodes select per row. */
+static double values_many_ns(const AttnArgs &a, int ct, long long wgs) {
+    const bool four = ct == 4;
+    double ns = four ? 12000 : 7000;
+    for (long long w0 = 0; w0 < wgs; w0 += 512) {
+        const double rows = a.g.nr_max - (a.g.chain ? (double)a.T * w0 / wgs : 0.0);
+        ns += (wgs - w0 <= 256 ? (four ? 64 : 42) : (four ? 79 : 49)) * rows + (w0 ? 2000 : 0);
+        if (!a.g.chain) ns += (four ? 120 : 75) * a.T;
+    }
+    return ns;
+}
+
+bool values_many(const AttnArgs &a, double other_ns, hipStream_t st) {
     if (a.hd % 64 || (!a.g.chain && a.T > VM_TREE)) return false;
     const int grp = a.H / a.Hkv, nd = a.hd / 64;
-    /* from two workgroups a CU on (rows of 64 heads x 128 columns from 64 tokens on): fewer
-     * leave a SIMD a lone wave, which waits for each product's latency (9 tokens of 128
-     * latent heads 257 us against 170 with the summing waves of k_attn_values_w, 85 tokens
-     * of 32 heads at 2048 140 against 58). A prefill of mostly its own tokens has rows of
-     * very different lengths, which more and smaller workgroups even out */
     auto wgs = [&](int ct) { return ((long long)a.T * grp + 16 * ct - 1) / (16 * ct) * a.Hkv * nd; };
-    if (wgs(4) < 512) return false;
-    if (a.g.chain && 2 * a.T > a.g.nr_max && wgs(4) < 1024) k_values_many<2><<<(int)wgs(2), 256, 0, st>>>(a);
+    /* The line lies where the times cross: a workgroup here takes the latency of its rows
+     * however few there are, where the others split by token and head. Measured, these with 2
+     * and 4 column tiles / the others, us a launch. Groups of 8 of 32 heads of 128: at 0, 128
+     * tokens 12.8, 18.7 / 12.3, 256 19.4, 27.7 / 26.6, 512 41.9, 46.7 / 61.5; at 4000, 128 tokens
+     * 171, 262 / 131, 256 200, 271 / 257, 320 399, 325 / 328, 464 445, 353 / 498, 512 455, 367 /
+     * 535; trees at 2047 of 85 103, 154 / 55, 512 305, 270 / 265. 32 single heads: at 0, 64 tokens
+     * 11, 19 / 58, at 4000 196, 289 / 469; tree of 85 at 2047 108, 157 / 366. 128 latent heads: at
+     * 4000, 9 tokens 195, 256 / 160, 32 386, 316 / 493. */
+    const double t2 = values_many_ns(a, 2, wgs(2)), t4 = values_many_ns(a, 4, wgs(4));
+    if (std::min(t2, t4) >= 0.97 * other_ns) return false;
+    if (t2 < t4) k_values_many<2><<<(int)wgs(2), 256, 0, st>>>(a);
     else k_values_many<4><<<(int)wgs(4), 256, 0, st>>>(a);
     return true;
 }
