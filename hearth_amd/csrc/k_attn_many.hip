@@ -438,7 +438,16 @@ namespace hxl {
 
 bool scores_many(const AttnArgs &a, hipStream_t st) {
     const int grp = a.H / a.Hkv;
-    if (a.post || a.T * grp < 64 || (a.hd != 64 && a.hd != 128 && a.hd != 256 && a.hd != 512)) return false;
+    if (a.post || (a.hd != 64 && a.hd != 128 && a.hd != 256 && a.hd != 512)) return false;
+    /* A workgroup takes the latency of its slot tiles however few its rows are; the others read
+     * the rows of K once a token. Measured, these / the others, us a launch: latent rows (with
+     * the RoPE term) of 16 heads, one token at 0 15 / 33, at 1000 30 / 39, at 4000 31 / 41, of 4
+     * heads, one token at 4000 30 / 23, 9 tokens 32 / 37; single heads of 128, 32 tokens at 0
+     * 6.4 / 7.2, at 1000 15 / 40 (17 at 0 level, but the whole call 1% slower); groups of 2 of
+     * 256, 32 tokens at 0 9.4 / 6.5, at 1000 16 / 40; groups of 8 of 128, 17 tokens at 0 7.9 /
+     * 6.8, at 4000 29.5 / 26.5, 24 at 4000 30 / 36 */
+    const bool few = a.T * grp < 64 && !(a.hd == 512 && grp >= 16) && !(a.hd <= 128 && a.T >= 32);
+    if (few) return false;
     const bool pe = a.qpe != nullptr;
     if (pe && (a.hd != 512 || a.qpe_ld % 4 || ((uintptr_t)a.qpe & 15))) return false;
     if ((64LL / grp + 2) * a.H * a.ldS >= 1LL << 32) return false;

@@ -1,9 +1,10 @@
-"""Which value kernel sums a call (the summing waves of k_attn.hip, or k_values_many with two or
-four column tiles) is decided by expected times: shapes that the line now gives to each, bit for
-bit against the oracle. Single heads, groups of 4 and 8, 64 / 128 / 192 columns, latent rows of
-256 and 512; chains and trees of few and of many tokens, from empty and after a context; and the
-device loop's padded steps of 21 tokens. The outputs have no tolerance: every sum's order is
-fixed."""
+"""Which score and value kernels a call takes. The value kernel (the summing waves of
+k_attn.hip, or k_values_many with two or four column tiles) is decided by expected times, the
+score kernel (k_scores_many or the others) by rows and tokens: shapes on both sides of the
+lines, bit for bit against the oracle. Single heads, groups of 4 and 8, 64 / 128 / 192 columns,
+latent rows of 256 and 512 and of 16 and 48 heads; chains and trees of few and of many tokens,
+from empty and after a context; and the device loop's padded steps of 21 tokens. The outputs
+have no tolerance: every sum's order is fixed."""
 from __future__ import annotations
 
 import dataclasses
@@ -27,6 +28,7 @@ LATENT256 = dataclasses.replace(container.TINY_MLA_NOQ, d_model=256, n_experts=4
 LATENT512 = dataclasses.replace(container.TINY_DSV3, n_layers=2, d_model=256, n_experts=8, n_group=2, topk_group=1, top_k=2,
                                 expert_ffn=128, shared_ffn=128, dense_ffn=128, vocab=512, n_heads=48, n_kv_heads=48,
                                 kv_lora=512)
+LATENT16 = dataclasses.replace(LATENT512, n_heads=16, n_kv_heads=16)
 
 
 def _bits(x):
@@ -38,8 +40,8 @@ def _bits(x):
 # LATENT256; the summing waves: the others
 @pytest.mark.parametrize("shape,lens,trees", [(SINGLE, (17, 33, 64, 2, 130), (21, 70)), (H64, (100, 40, 200, 9), (33, 129)),
                                               (H192, (31, 500, 20), (100,)), (LATENT256, (24, 48, 129, 3), (40, 90)),
-                                              (LATENT512, (13, 260, 50, 18), (21, 64))],
-                         ids=["single", "h64", "h192", "latent256", "latent512"])
+                                              (LATENT512, (13, 260, 50, 18), (21, 64)), (LATENT16, (1, 2, 3, 40, 1), (2, 3))],
+                         ids=["single", "h64", "h192", "latent256", "latent512", "latent16"])
 def test_value_sums(tmp_path, shape, lens, trees):
     O.gpu_numerics()
     path = container.make_tiny(tmp_path / "m.hearth", _native.quantize, seed=23, shape=shape)
