@@ -8,7 +8,8 @@
  * the token's rows. The order of each sum is fixed and each product is rounded before it
  * is added, so the sums stay on the vector units. The products come from
  * v_mfma_f32_16x16x1_4b_f32 with a zero accumulator: one multiplication per output, rounded
- * once (subnormals kept), exactly fmul. What that buys is the operands: an instruction
+ * once, subnormals kept: fmul (the sign of a zero product is not relied on: every sum here
+ * starts at +0, which neither zero changes). What that buys is the operands: an instruction
  * takes one register of rows and one of columns for 1024 products, where the vector units
  * would need one operand of each product broadcast over the lanes -- by DPP 6 cycles an
  * instruction against 2 (32 terms a clock and CU), from LDS 4 bytes a lane. The MFMA and

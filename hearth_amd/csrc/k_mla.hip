@@ -76,7 +76,7 @@ __device__ __forceinline__ int seg_bytes(int dt) { return dt == 3 ? 66 : dt == 4
  * and 16 CT columns at a time (the four waves are CT token tiles of the 64 columns).
  *
  * Every term is a rounded product and an add in order. The products come from
- * v_mfma_f32_16x16x1_4b_f32 with a zero accumulator (rounded once, exactly fmul): one
+ * v_mfma_f32_16x16x1_4b_f32 with a zero accumulator (rounded once, subnormals kept): one
  * register of q and one of W give the 1024 products of 16 tokens, 16 columns and 4 rows n,
  * so that the adds are all that is left to the vector units. Bound by products and adds for
  * many tokens, by staging and dequantization for few. Before (a column a lane, the weight
