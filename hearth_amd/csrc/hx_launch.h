@@ -24,7 +24,7 @@ struct GemmArgs {
     GemmSeg seg[4];
     int nseg;
     Act a;             /* activations of tokens [0, T) */
-    int T, t0;
+    int T;
     /* device [1] or null: tokens t >= *live are padding, whose output rows the split-K
      * product leaves unwritten (nothing reads them) */
     const int *live;

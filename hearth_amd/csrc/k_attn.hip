@@ -559,8 +559,10 @@ constexpr int TV_PS = 4;                /* p ring slots of k_attn_values_w */
 constexpr int TV_PS3 = 5;               /* and of k_attn_values, which publishes a tile earlier */
 constexpr int TV_THREADS = 768;         /* 4 summing + 8 loader waves */
 constexpr int TV_SUM = 4, TV_LOAD = 8;  /* summing waves (one head each), loader waves */
-/* the staging map below: loader wave lw owns tile rows 16 lw .. 16 lw + 15 (lane % 16)
- * and p half lw % 2 of head lw / 2; lane / 16 picks 4 of each 16 columns */
+/* the staging map of k_attn_values: loader wave lw owns tile rows 16 lw .. 16 lw + 15, lane /
+ * 16 a row of each 4, lane % 16 four columns, and p half lw % 2 of head lw / 2 (k_attn_values_w
+ * has a map of its own over the same blocks: lane % 16 the row, lane / 16 four of each 16
+ * columns, the columns in order) */
 static_assert(TV_THREADS == 64 * (TV_SUM + TV_LOAD), "k_attn_values: 4 summing + 8 loader waves");
 static_assert(TV_ROWS == 16 * TV_LOAD, "k_attn_values: each loader wave stages 16 rows of a tile");
 static_assert(TV_LOAD == 2 * TV_SUM && TV_ROWS == 2 * 64, "k_attn_values: two 64-row p halves per summed head");

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(512) void k_gemm_sk(GemmArgs args, int ntok) {
      * with short drafts. */
     const int lv = args.live ? *args.live : args.T;
     const int T = lv < args.T ? lv : args.T;
-    for (int t0 = args.t0; t0 < T; t0 += ntok) {
+    for (int t0 = 0; t0 < T; t0 += ntok) {
         tile_terms<DT, 1>(&sg.m, rt, args.a, t0, T, ntok, [](int t) { return t; }, p0, p1, P, 0);
         __syncthreads();
         const int nc = T - t0 < ntok ? T - t0 : ntok;

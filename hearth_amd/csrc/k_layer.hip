@@ -645,7 +645,7 @@ __global__ __launch_bounds__(1024) void k_route_bucket(RouteArgs a) {
  * workgroup. Wave t routes token t: scores and weights as k_route_rank; the K experts by
  * K rounds of a wave maximum of the 32-bit order keys of the selection values, the winner
  * being the lowest expert index that holds the maximum (ballots in index order), which is
- * the reference's order (ranks_before). Each choice sets the token's bit in its expert's token mask, so
+ * the order of rank_key. Each choice sets the token's bit in its expert's token mask, so
  * the bucketing needs no counting pass: an expert's pair count is the popcount of its
  * mask, and a pair's place among its expert's pairs (tokens ascending, model.c:1030-1035)
  * the popcount of the mask bits below its token (a token's K experts are distinct:

@@ -271,10 +271,11 @@ __device__ __forceinline__ bool mm_item(const MoeArgs &a, int item, int G, int &
 }
 
 /* gate/up of 64 rows of one active expert (one block of the down product's K) for its n
- * tokens t0 .. t0 + 16 NT - 1 (an item): mid = silu(g) * u (NUMERICS §4, quant.c:644-649), then NUMERICS
- * §2 of the block, straight into the down product's activations. */
-template <int DT, int NT>
+ * tokens t0 .. t0 + 15 (an item): mid = silu(g) * u (NUMERICS §4, quant.c:644-649), then
+ * NUMERICS §2 of the block, straight into the down product's activations. */
+template <int DT>
 __global__ __launch_bounds__(256, 2) void k_mm_gateup(MoeArgs a) {
+    constexpr int NT = 1;
     __shared__ __attribute__((aligned(16))) MmStage<2, NT> st[2];
     __shared__ unsigned long long tab[32];
     const int nrg = a.F / 64;
@@ -392,7 +393,7 @@ void mm_gateup(const MoeArgs &a, int n_slots, hipStream_t st, hipEvent_t ev0, hi
     const bool q4 = a.dtype_mask & (1 << 4), q8 = a.dtype_mask & (1 << 3);
     const dim3 grid(mm_items(a, n_slots, 1) * (a.F / 64));
 #define MM_L(DT_, E0, E1) \
-    hipExtLaunchKernelGGL((k_mm_gateup<DT_, 1>), grid, dim3(256), 0, st, E0, E1, 0u, a);
+    hipExtLaunchKernelGGL(k_mm_gateup<DT_>, grid, dim3(256), 0, st, E0, E1, 0u, a);
     if (q4) { MM_L(4, ev0, q8 ? nullptr : ev1) }
     if (q8) { MM_L(3, q4 ? nullptr : ev0, ev1) }
 #undef MM_L

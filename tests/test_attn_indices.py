@@ -11,7 +11,7 @@ prefill geometries the GPU tests run, and must stay in range:
   value loop (rows jl .. nk - 1);
 - k_attn_values / k_attn_values_w: the tree loads (row v clamped to nr - 1, anc_s index
   v - pos0 when v > pos0, the source row pos0 + anc or v itself) of every tile the
-  three-deep load pipeline issues, and anc_s's size.
+  load pipelines issue, and anc_s's size.
 
 A geometry is what hearth_engine::run_geometry uploads: depth[t] (t for a chain, the
 parent's depth + 1 for a tree) and anc[t][0..depth[t]] (the path from node 0 to t). The
@@ -113,17 +113,17 @@ def check_chunk(pos0, depth, anc, chain, H, Hkv, hd, cap, kshared_of=None):
     return seen
 
 
-def check_values(pos0, depth, anc, chain, cap, rows_per_tile, loaders, clamp=True):
-    """The loads of k_attn_values (rows_per_tile 128, 8 loader waves) or
-    k_attn_values_w (ROWS = 16 NL) for every token: tiles 0 .. ntiles + 2 of the load
-    pipeline (three loads ahead; the last steps load nothing, the main loop stops at
-    i + 3 <= ntiles, so the highest tile loaded is ntiles + 2)."""
+def check_values(pos0, depth, anc, chain, cap, rows_per_tile, loaders, ahead, clamp=True):
+    """The loads of k_attn_values (rows_per_tile 128, 8 loader waves, step i loads tile
+    i + 4) or k_attn_values_w (ROWS = 16 NL, step i loads tile i + 3) for every token: the
+    prologue loads tiles 0 .. ahead - 1, the last steps load nothing, the main loop stops at
+    i + 3 <= ntiles, so the highest tile loaded is at most ntiles - 1 + ahead."""
     for t in range(len(depth)):
         dep = int(depth[t])
         nr = pos0 + dep + 1
         assert dep < MAX_ANC   # anc_s[MAX_ANC]
         ntiles = (nr + rows_per_tile - 1) // rows_per_tile
-        hi_tile = ntiles + 2 if ntiles >= 3 else 2
+        hi_tile = ntiles - 1 + ahead if ntiles >= 3 else ahead - 1
         lw = np.arange(loaders)[:, None]
         r = np.arange(16)[None, :]
         for i in range(hi_tile + 1):
@@ -185,8 +185,8 @@ def test_attention_indices_in_range(model, geo):
     chain = parent is None or all(parent[i] == i - 1 for i in range(T))
     if chunked_ok(hd, H // Hkv):
         assert check_chunk(pos0, depth, anc, chain, H, Hkv, hd, cap) > 0
-    check_values(pos0, depth, anc, chain, cap, TV_ROWS, TV_LOAD)
-    check_values(pos0, depth, anc, chain, cap, 64, 4)   # k_attn_values_w<., 4, ., 64>
+    check_values(pos0, depth, anc, chain, cap, TV_ROWS, TV_LOAD, 4)
+    check_values(pos0, depth, anc, chain, cap, 64, 4, 3)   # k_attn_values_w<., 4, ., 64>
 
 
 def test_checks_catch_planted_mistakes():
@@ -201,9 +201,9 @@ def test_checks_catch_planted_mistakes():
         check_chunk(pos0, depth, anc, True, 32, 4, 128, 4104, kshared_of=lambda r0: 0)
     parent = [-1, 0, 0, 1, 1, 2, 3]
     depth, anc = geometry(7, parent)
-    check_values(49, depth, anc, False, 1024, TV_ROWS, TV_LOAD)
+    check_values(49, depth, anc, False, 1024, TV_ROWS, TV_LOAD, 4)
     with pytest.raises(AssertionError):
-        check_values(49, depth, anc, False, 1024, TV_ROWS, TV_LOAD, clamp=False)
+        check_values(49, depth, anc, False, 1024, TV_ROWS, TV_LOAD, 4, clamp=False)
 
 
 def test_chunked_ok_bounds_items():

@@ -1,14 +1,15 @@
 """The value kernels' load counts in this build's own AMD assembly.
 
 k_attn_values and k_attn_values_w (hearth_amd/csrc/k_attn.hip) keep three V tiles in
-flight and publish tile i + 1 after `s_waitcnt vmcnt(WV)` with WV = 2 * (4 + PL): the
-wait is right only if every tile issues exactly WV / 2 vector-memory loads (4 16-byte V
-loads and PL LDS-direct p loads), so that the WV loads still outstanding are exactly
-those of the two tiles after it. A compiler that dropped or merged a load would make the
-wait release a tile whose loads are still in flight, with no build error. This test
-compiles k_attn.hip to gfx950 assembly with the library's flags and checks, along each
-kernel's code, that the first vmcnt(WV) of a pipeline follows 3 WV / 2 loads (the three
-tiles of the prologue) and every later one WV / 2 loads (the tile each step issues).
+flight. After `s_waitcnt vmcnt(WV)`, WV = 2 * (4 + PL), a loader wave of k_attn_values stores
+tile i + 2, one of k_attn_values_w tile i + 1, and the next barrier publishes it: the wait is
+right only if every tile issues exactly WV / 2 vector-memory loads (4 16-byte V loads and PL
+LDS-direct p loads), so that the WV loads still outstanding are exactly those of the two
+tiles after it. A compiler that dropped or merged a load would make the wait release a tile
+whose loads are still in flight, with no build error. This test compiles k_attn.hip to
+gfx950 assembly with the library's flags and checks, along each kernel's code, that the
+first vmcnt(WV) of a pipeline follows 3 WV / 2 loads (the three tiles of the prologue) and
+every later one WV / 2 loads (the tile each step issues).
 Waits for fewer loads (vmcnt(0), the geometry's own loads) start a new pipeline; waits
 for more loads than WV are weaker than the pipeline's and are skipped.
 """
