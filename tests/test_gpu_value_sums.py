@@ -29,6 +29,7 @@ LATENT512 = dataclasses.replace(container.TINY_DSV3, n_layers=2, d_model=256, n_
                                 expert_ffn=128, shared_ffn=128, dense_ffn=128, vocab=512, n_heads=48, n_kv_heads=48,
                                 kv_lora=512)
 LATENT16 = dataclasses.replace(LATENT512, n_heads=16, n_kv_heads=16)
+ROPE32 = dataclasses.replace(LATENT256, n_heads=16, n_kv_heads=16, kv_lora=512)   # the RoPE term a pass of its own
 
 
 def _bits(x):
@@ -40,8 +41,9 @@ def _bits(x):
 # LATENT256; the summing waves: the others
 @pytest.mark.parametrize("shape,lens,trees", [(SINGLE, (17, 33, 64, 2, 130), (21, 70)), (H64, (100, 40, 200, 9), (33, 129)),
                                               (H192, (31, 500, 20), (100,)), (LATENT256, (24, 48, 129, 3), (40, 90)),
-                                              (LATENT512, (13, 260, 50, 18), (21, 64)), (LATENT16, (1, 2, 3, 40, 1), (2, 3))],
-                         ids=["single", "h64", "h192", "latent256", "latent512", "latent16"])
+                                              (LATENT512, (13, 260, 50, 18), (21, 64)), (LATENT16, (1, 2, 3, 40, 1), (2, 3)),
+                                              (ROPE32, (1, 3, 20, 1), (4,))],
+                         ids=["single", "h64", "h192", "latent256", "latent512", "latent16", "rope32"])
 def test_value_sums(tmp_path, shape, lens, trees):
     O.gpu_numerics()
     path = container.make_tiny(tmp_path / "m.hearth", _native.quantize, seed=23, shape=shape)
